@@ -231,7 +231,7 @@ DecodePlan make_plan(int B, int Hq, int Hkv, int d, int max_len, bool aligned, b
     }
     p.fast = p.kernel != kvq::Kernel::Generic;
     p.tile = tile;
-    p.nsg = p.fast ? G / p.sg : G;
+    p.nsg = p.fast ? (G + p.sg - 1) / p.sg : G;
     const long units = p.fast ? static_cast<long>(B) * Hkv * p.nsg : static_cast<long>(B) * Hq;
     const int gran = p.fast ? tile : 64;
     max_len = std::max(max_len, 1);

@@ -1,10 +1,12 @@
 // kvq_decode_mfma.hip -- grouped-query decode attention on gfx950 matrix cores.
 //
 // For G query heads sharing a kv head the per-token work is a small dense
-// contraction (QK: [G x D] x [D x T], PV: [G x T] x [T x D]), so with G = 4
-// or 8 it runs on MFMA instead of per-lane FMAs.  Same math and result
+// contraction (QK: [G x D] x [D x T], PV: [G x T] x [T x D]), so with two or
+// more heads it runs on MFMA instead of per-lane FMAs.  Same math and result
 // contract as decode_fast (the reference's cpu_reference per query head,
-// kv_cache/KV_int8_split_optimized.cu:385-437); head dim D = 64 or 128.
+// kv_cache/KV_int8_split_optimized.cu:385-437).  The kernels are built for
+// D = 64 or 128 dims and G = 4 or 8 heads; PAD instances take any head dim
+// that is a multiple of 16 up to D and any head count up to G.
 //
 // One workgroup (4 waves) per (sequence split, batch, kv head, group of G
 // query heads); each wave walks 32-token tiles with its own online-softmax
@@ -15,12 +17,14 @@
 //   64-dim block); no dequantisation instruction touches K.  q is held as three
 //   balanced int8 limbs of a 22-bit fixed-point value per head (q*2^E rounded
 //   once, |error| <= 2^-23 * max|q|), one MFMA column block per limb; the int32
-//   products are exact, and dot = ((C0*2^16 + C1*2^8) + C2) * 2^-E.
+//   products are exact, and dot = ((C0*2^16 + C1*2^8) + C2) * 2^-E.  PAD: four
+//   limbs, 30 bits, which hold every fp32 q to 2^-31 * max|q| (q_limbs).
 //   MFMA rows n = 0..15 all carry head n % G (duplicates are free).
 // * softmax: the running max m of s = (dot * k_scale) * softmax_scale * log2 e
 //   gives p = exp2(s - m) and the denominator; the PV weights are
 //   w = p * v_scale * 2^15 / vref, with vref the running max of |v_scale|, so
-//   |w| <= 2^15 whatever the scale magnitudes.  A tile that raises m or vref
+//   |w| <= 2^15 whatever the scale magnitudes (PAD: vref is the power of two
+//   above that max, so scaling by it rounds nothing).  A tile that raises m or vref
 //   rescales the accumulator once (skipped when no row of the wave changed).
 // * PV on v_mfma_f32_16x16x32_f16 computing O^T[dim, row] += V^T P: the
 //   weights are split into f16 hi + lo rows (rows n < G.. hold hi, the next G
@@ -35,6 +39,7 @@
 // * fused append: the new token is quantised by the one wave whose last tile
 //   holds token length-1 (its fp32 loads were issued at kernel start) and
 //   substituted from LDS into that tile.
+#include <limits.h>
 #include <math.h>
 
 #include "kvq_device.hpp"
@@ -53,7 +58,7 @@ typedef __attribute__((address_space(3))) i32x2 lds_i32x2;
 
 constexpr int kMWaves = kMfmaWaves;  // waves per workgroup
 constexpr int kMTile = kMfmaTile;  // tokens per wave tile
-constexpr float kPScale = 32768.0f;  // PV weights are formed in [-2^15, 2^15] before the f16 split
+constexpr float kPScale = 32768.0f;  // PV weights are formed in (-2^15, 2^15) before the f16 split
 constexpr int kMBStep = kMTile * kMWaves;
 
 // 8 signed bytes -> 8 f16 (exact): bias each byte to unsigned, place it under
@@ -71,6 +76,11 @@ __device__ __forceinline__ f16x8 i8x8_to_f16(i32x2 v) {
     const f16x2 h2 = __builtin_bit_cast(f16x2, w2) - bias;
     const f16x2 h3 = __builtin_bit_cast(f16x2, w3) - bias;
     return f16x8{h0.x, h0.y, h1.x, h1.y, h2.x, h2.y, h3.x, h3.y};
+}
+
+// The power of two above x >= 0 (0 for 0): dividing by it and multiplying back is exact.
+__device__ __forceinline__ float pow2_above(float x) {
+    return x > 0.0f ? __uint_as_float((__float_as_uint(x) & 0x7f800000u) + 0x00800000u) : 0.0f;
 }
 
 __device__ __forceinline__ int pack_bytes(const int* b) {
@@ -92,11 +102,38 @@ __device__ __forceinline__ int v_slot(int p, int rw) {
     else return p ^ (((rw >> 2) & 1) | ((rw >> 3) & 2));
 }
 
-template <int D, int G, bool PAGED, bool FIT>
+// Byte offset of a load that must read zeros and touch no memory (at or past
+// the end of every resource here: a sequence's rows are below 2^31 bytes).
+constexpr int kOobOffset = INT_MIN;
+
+// int8 limbs of a q element: 8 * limbs - 2 bits of fixed point.  The PAD
+// shapes ran on fp32 FMAs before; with three limbs their error against 64 bits
+// was 4.2e-7 (6 heads, d = 128, 1K-8K tokens) where the FMA kernel's is 2.3e-7,
+// with four and the exact vref 2.0e-7.  The fourth limb costs 0.3-0.4 us per
+// launch there (4 more MFMAs per tile); in the tile-stream kernel without PAD
+// its 22 registers spill (B16 Hq32/Hkv8 L 1K-8K: 36.8 against 32.0 us).
+template <bool PAD>
+constexpr int q_limbs() { return PAD ? 4 : 3; }
+
+// PAD: the head dim a.d is a multiple of 16 below D, and / or the workgroup has
+// fewer than G heads (a.sgh, fewer still in the last group).  Rows are read at
+// their own stride; the 16-byte pieces past a.d are loaded out of bounds, so
+// they cost no memory traffic and arrive as zeros (zero q limbs, zero V
+// columns), and head slots past the group's repeat its last head and store
+// nothing.  The work per tile is that of <D, G>, but the tile loop is bound by
+// memory: one pass over K and V, where decode_fast rereads them once per 1, 2
+// or 4 heads and decode_generic (other head dims) once per head in byte loads.
+// Before / after at B16 Hkv8 L 1K-8K d128: 6 heads per kv head 118 / 38 us, 7
+// heads 171 / 43 us, 12 heads (two groups of 6) 95 / 68 us; B64 2 heads L
+// 300-4K 99 / 69 us; B8 3 heads d96 L 500-3K 1417 / 20 us.
+
+template <int D, int G, bool PAGED, bool FIT, bool PAD>
 __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(2))) void decode_mfma(
     const DecodeArgs a) {
     static_assert(G == 4 || G == 8, "heads per workgroup");
     static_assert(D == 64 || D == 128, "head dims of the matrix-core decode kernel");
+    constexpr int kLimbs = q_limbs<PAD>();
+    constexpr int kQBits = 8 * kLimbs - 2;
     constexpr int NJ = D / 64;            // 64-dim blocks of a K row (QK k-steps, q limb blocks)
     constexpr int NB = D / 16;            // 16-byte pieces of a row (PV blocks)
     constexpr int RPLV = kWave / NB;      // V rows one tile load instruction covers
@@ -140,14 +177,17 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
     const int sgi = unit - bh * a.nsg;
     const int b = bh / a.Hkv;
     const int kvh = bh - b * a.Hkv;
-    const int hq0 = kvh * a.G + sgi * G;
+    const int d = PAD ? a.d : D;
+    const int sgh = PAD ? a.sgh : G;                        // heads per group
+    const int hc = PAD ? min(sgh, a.G - sgi * sgh) : G;     // heads of this group
+    const int hq0 = kvh * a.G + sgi * sgh;
     const size_t bhq0 = static_cast<size_t>(b) * a.Hq + hq0;
     const int len = w.len;
     const int split = w.split;
     const int nsplit = w.nsplit;
 
     if (len == 0) {
-        for (int i = threadIdx.x; i < G * D; i += blockDim.x) a.out[bhq0 * D + i] = 0.0f;
+        for (int i = threadIdx.x; i < hc * d; i += blockDim.x) a.out[bhq0 * d + i] = 0.0f;
         return;
     }
 
@@ -163,21 +203,23 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
     const bool own_new = app && ((tnew - t0) / kMTile) % kMWaves == wave;
     float xnew[NE];
 #pragma unroll
-    for (int j = 0; j < NE; j++)
-        xnew[j] = own_new ? (j < NJ ? a.k_new : a.v_new)[static_cast<size_t>(bh) * D + ((lane + kWave * j) & (D - 1))]
-                          : 0.0f;
+    for (int j = 0; j < NE; j++) {
+        const int e = (lane + kWave * j) & (D - 1);
+        xnew[j] = own_new && (!PAD || e < d) ? (j < NJ ? a.k_new : a.v_new)[static_cast<size_t>(bh) * d + e] : 0.0f;
+    }
 
     // q of head (r % G) as int8 limbs in the QK B operand layout:
     // qb[j][limb] holds dims 64j + 16g + [0,16).
-    const int hrow = r % G;
+    const int hrow = PAD ? min(r % G, hc - 1) : r % G;
     float qv[16 * NJ];
     {
-        const float* qp = a.q + (bhq0 + hrow) * D + 16 * g;
+        const float* qp = a.q + (bhq0 + hrow) * d + 16 * g;
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
 #pragma unroll
             for (int i4 = 0; i4 < 4; i4++) {
-                const float4 x = *reinterpret_cast<const float4*>(qp + 64 * j + 4 * i4);
+                const float4 x = !PAD || 64 * j + 16 * g < d ? *reinterpret_cast<const float4*>(qp + 64 * j + 4 * i4)
+                                                             : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                 qv[16 * j + 4 * i4] = x.x;
                 qv[16 * j + 4 * i4 + 1] = x.y;
                 qv[16 * j + 4 * i4 + 2] = x.z;
@@ -188,7 +230,7 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
     // The limbs are formed after the first tile's loads are issued (their
     // latency overlaps this work); qs turns an integer dot into a score in
     // log2 units (after x k_scale).
-    i32x4 qb[NJ][3];
+    i32x4 qb[NJ][kLimbs];
     float qs = 0.0f;
     auto prepare_q = [&]() {
         float qmax = 0.0f;
@@ -198,23 +240,23 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
         qmax = fmaxf(qmax, __shfl_xor(qmax, 32));
         int qexp = 0;
         frexpf(qmax, &qexp);  // qmax < 2^qexp
-        const int E = qmax > 0.0f ? min(max(22 - qexp, -100), 126) : 0;
+        const int E = qmax > 0.0f ? min(max(kQBits - qexp, -100), 126) : 0;
         qs = ldexpf(1.0f, -E) * a.scale_log2;
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
-            int limb[3][16];
+            int limb[kLimbs][16];
 #pragma unroll
             for (int i = 0; i < 16; i++) {
-                const int Q = static_cast<int>(__builtin_rintf(ldexpf(qv[16 * j + i], E)));
-                const int l2 = ((Q + 128) & 255) - 128;
-                const int Q1 = (Q - l2) >> 8;
-                const int l1 = ((Q1 + 128) & 255) - 128;
-                limb[0][i] = (Q1 - l1) >> 8;
-                limb[1][i] = l1;
-                limb[2][i] = l2;
+                int Q = static_cast<int>(__builtin_rintf(ldexpf(qv[16 * j + i], E)));
+#pragma unroll
+                for (int lb = kLimbs - 1; lb > 0; lb--) {
+                    limb[lb][i] = ((Q + 128) & 255) - 128;
+                    Q = (Q - limb[lb][i]) >> 8;
+                }
+                limb[0][i] = Q;
             }
 #pragma unroll
-            for (int lb = 0; lb < 3; lb++)
+            for (int lb = 0; lb < kLimbs; lb++)
                 qb[j][lb] = i32x4{pack_bytes(&limb[lb][0]), pack_bytes(&limb[lb][4]), pack_bytes(&limb[lb][8]),
                                   pack_bytes(&limb[lb][12])};
         }
@@ -236,8 +278,8 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
     // reads past the capacity return 0.  A paged cache gets resources per
     // tile instead (below).
     const unsigned cap = static_cast<unsigned>(a.cap);
-    const buf_rsrc kres = make_rsrc(a.k + row0 * D, cap * D);
-    const buf_rsrc vres = make_rsrc(a.v + row0 * D, cap * D);
+    const buf_rsrc kres = make_rsrc(a.k + row0 * d, cap * d);
+    const buf_rsrc vres = make_rsrc(a.v + row0 * d, cap * d);
     const buf_rsrc ksres = make_rsrc(a.ks + row0, cap * 4u);
     const buf_rsrc vsres = make_rsrc(a.vs + row0, cap * 4u);
 
@@ -268,8 +310,9 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
         if (sgi == 0) {
             if (lane < 2 * NB) {
                 const int row = lane / NB, piece = lane % NB;
-                *reinterpret_cast<int4*>((row ? a.v : a.k) + rnew * D + 16 * piece) =
-                    *reinterpret_cast<const int4*>(&s_newq[row][16 * piece]);
+                if (!PAD || 16 * piece < d)
+                    *reinterpret_cast<int4*>((row ? a.v : a.k) + rnew * d + 16 * piece) =
+                        *reinterpret_cast<const int4*>(&s_newq[row][16 * piece]);
             }
             if (lane == 0) {
                 a.ks[rnew] = newks;
@@ -293,6 +336,14 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
     const int kvo = r * D + 16 * g;
     const int vvo = (lane / NB) * D + 16 * (lane % NB);
     const int svo = 16 * g;
+    auto k_off = [&](int s, int j) {
+        if constexpr (!PAD) return kvo + s * 16 * D + 64 * j;
+        else return 64 * j + 16 * g < d ? (r + 16 * s) * d + 16 * g + 64 * j : kOobOffset;
+    };
+    auto v_off = [&](int c) {
+        if constexpr (!PAD) return vvo + c * RPLV * D;
+        else return 16 * (lane % NB) < d ? (lane / NB + c * RPLV) * d + 16 * (lane % NB) : kOobOffset;
+    };
     // Paged: each tile's page id comes from the block table one tile ahead,
     // by a vector load issued before the previous tile's K/V loads, so a
     // tile's loads wait only for that id (in-order vector-memory counter),
@@ -311,7 +362,7 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
     if constexpr (PAGED) pg_next = fetch_page(0);
     auto load_tile = [&](Tile& T, int it) {
         const int base = wbase + it * kMBStep;
-        int ko = base * D;
+        int ko = base * d;
         int so = base * 4;
         buf_rsrc kr = kres, vr = vres, ksr = ksres, vsr = vsres;
         if constexpr (PAGED) {
@@ -321,8 +372,8 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
             pg_next = fetch_page(it + 1);
             const size_t rp = (static_cast<size_t>(page) * a.Hkv + kvh) * a.pages.size + (base & (a.pages.size - 1));
             const unsigned rem = static_cast<unsigned>(a.pages.size - (base & (a.pages.size - 1)));
-            kr = make_rsrc(a.k + rp * D, rem * D);
-            vr = make_rsrc(a.v + rp * D, rem * D);
+            kr = make_rsrc(a.k + rp * d, rem * d);
+            vr = make_rsrc(a.v + rp * d, rem * d);
             ksr = make_rsrc(a.ks + rp, rem * 4u);
             vsr = make_rsrc(a.vs + rp, rem * 4u);
             ko = so = 0;
@@ -330,11 +381,11 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
         for (int s = 0; s < 2; s++) {
 #pragma unroll
-            for (int j = 0; j < NJ; j++) T.ka[s][j] = buffer_load16_stream(kr, kvo + s * 16 * D + 64 * j, ko);
+            for (int j = 0; j < NJ; j++) T.ka[s][j] = buffer_load16_stream(kr, k_off(s, j), ko);
         }
 #pragma unroll
         for (int c = 0; c < NV; c++) {
-            const v4i_t x = buffer_load16_stream(vr, vvo + c * RPLV * D, ko);
+            const v4i_t x = buffer_load16_stream(vr, v_off(c), ko);
             T.v[c] = make_int4(x.x, x.y, x.z, x.w);
         }
 #pragma unroll
@@ -383,11 +434,11 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
     // check_tail: the tile may reach past tend (only a wave's last tile can).
     auto compute = [&](const Tile& T, int base, const int8_t* vt, bool check_tail) {
         // QK: C[token 4g + i][row r] per sub-tile and limb.
-        i32x4 cq[2][3];
+        i32x4 cq[2][kLimbs];
 #pragma unroll
         for (int s = 0; s < 2; s++) {
 #pragma unroll
-            for (int lb = 0; lb < 3; lb++) {
+            for (int lb = 0; lb < kLimbs; lb++) {
                 i32x4 c = i32x4{0, 0, 0, 0};
 #pragma unroll
                 for (int j = 0; j < NJ; j++) c = __builtin_amdgcn_mfma_i32_16x16x64_i8(T.ka[s][j], qb[j][lb], c, 0, 0, 0);
@@ -402,8 +453,9 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
         for (int s = 0; s < 2; s++) {
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const int low = (cq[s][1][i] << 8) + cq[s][2][i];
-                const float dot = static_cast<float>(cq[s][0][i]) * 65536.0f + static_cast<float>(low);
+                const int low = (cq[s][kLimbs - 2][i] << 8) + cq[s][kLimbs - 1][i];
+                const int high = kLimbs == 4 ? (cq[s][0][i] << 8) + cq[s][1][i] : cq[s][0][i];
+                const float dot = fmaf(static_cast<float>(high), 65536.0f, static_cast<float>(low));
                 sc[4 * s + i] = (dot * T.ks[s][i]) * qs;
                 vsv[4 * s + i] = T.vs[s][i];
             }
@@ -434,8 +486,8 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
         const float mn = fmaxf(m, mt);
         const float ms = mn == -INFINITY ? 0.0f : mn;
         const float alpha = fast_exp2(m - ms);
-        const float vn = fmaxf(vref, vmax);
-        const float rvn = vn > 0.0f ? __builtin_amdgcn_rcpf(vn) : 0.0f;  // v_rcp_f32, 1 ulp
+        const float vn = fmaxf(vref, PAD ? pow2_above(vmax) : vmax);
+        const float rvn = vn > 0.0f ? __builtin_amdgcn_rcpf(vn) : 0.0f;  // v_rcp_f32, 1 ulp (PAD: exact)
         const float f = vn > 0.0f ? alpha * (vref * rvn) : alpha;
         const float winv = kPScale * rvn;
         m = mn;
@@ -522,9 +574,10 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
     if (nsplit > 1) {
         map = rec_map(a, w, bhq0);
     }
-    for (int i = threadIdx.x; i < G * D; i += blockDim.x) {
+    for (int i = threadIdx.x; i < hc * D; i += blockDim.x) {
         const int h = i / D;
         const int dim = i - h * D;
+        if (PAD && dim >= d) continue;
         float M = -INFINITY;
 #pragma unroll
         for (int w = 0; w < kMWaves; w++) M = fmaxf(M, s_ml[w][h][0]);
@@ -538,7 +591,7 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
         }
         store_result(a, map, bhq0, h, dim, split, nsplit, M, L, A);
     }
-    finish_split<true>(a, unit, map, bhq0, G, nsplit, &s_last, s_u.merge);
+    finish_split<true>(a, unit, map, bhq0, hc, nsplit, &s_last, s_u.merge);
 }
 
 
@@ -593,18 +646,21 @@ __device__ __forceinline__ int flat_wave_of(const FlatSplit& f, int t) {  // the
 // ids w0 + b .. w0 + b + nrec - 1, record id r of head hq at row r * Hq + hq.
 // kWave / G lanes per head, each with D / 4 / (kWave / G) 16-byte columns:
 // a record's (m, l) load serves all of a lane's columns, and KR records per
-// round are loaded together with device-coherent buffer loads.
-template <int D, int G>
-__device__ inline void merge_wave_records(const DecodeArgs& a, int b, int w0, int nrec, int hq0, int lane) {
+// round are loaded together with device-coherent buffer loads.  PAD: hc <= G
+// heads of a.d <= D dims (the lanes of other heads and columns idle).
+template <int D, int G, bool PAD>
+__device__ inline void merge_wave_records(const DecodeArgs& a, int b, int w0, int nrec, int hq0, int hc, int lane) {
     constexpr int LPH = kWave / G;        // lanes per head
     constexpr int NC = D / 4 / LPH;       // 16-byte columns per lane
     constexpr int KR = NC <= 2 ? 16 : 8;  // records per round
+    const int d = PAD ? a.d : D;
     const int h = lane / LPH;
     const int c0 = lane - h * LPH;        // columns c0, c0 + LPH, ...
+    if (PAD && h >= hc) return;
     const size_t r0 = (static_cast<size_t>(w0) + b) * a.Hq + hq0;
-    const unsigned span = static_cast<unsigned>((nrec - 1) * a.Hq + G);
+    const unsigned span = static_cast<unsigned>((nrec - 1) * a.Hq + hc);
     const buf_rsrc mlr = make_rsrc(a.part_ml + r0 * 2, span * 8u);
-    const buf_rsrc accr = make_rsrc(a.part_acc + r0 * D, span * static_cast<unsigned>(D) * 4u);
+    const buf_rsrc accr = make_rsrc(a.part_acc + r0 * d, span * static_cast<unsigned>(d) * 4u);
     typedef int v2i_t __attribute__((ext_vector_type(2)));
     float M = -INFINITY, L = 0.0f;
     f32x4 A[NC];
@@ -620,7 +676,7 @@ __device__ inline void merge_wave_records(const DecodeArgs& a, int b, int w0, in
                 ml[k] = __builtin_amdgcn_raw_buffer_load_b64(mlr, rec * 8, 0, kCoherent);
 #pragma unroll
                 for (int j = 0; j < NC; j++)
-                    acc[k][j] = __builtin_amdgcn_raw_buffer_load_b128(accr, (rec * D + 4 * (c0 + j * LPH)) * 4, 0,
+                    acc[k][j] = __builtin_amdgcn_raw_buffer_load_b128(accr, (rec * d + 4 * (c0 + j * LPH)) * 4, 0,
                                                                       kCoherent);
             }
         }
@@ -644,19 +700,22 @@ __device__ inline void merge_wave_records(const DecodeArgs& a, int b, int w0, in
         }
     }
     const float rl = 1.0f / L;
-    float* o = a.out + (static_cast<size_t>(b) * a.Hq + hq0 + h) * D;
+    float* o = a.out + (static_cast<size_t>(b) * a.Hq + hq0 + h) * d;
 #pragma unroll
     for (int j = 0; j < NC; j++) {
+        if (PAD && 4 * (c0 + j * LPH) >= d) continue;
 #pragma unroll
         for (int i = 0; i < 4; i++) o[4 * (c0 + j * LPH) + i] = A[j][i] * rl;
     }
 }
 
-template <int D, int G, bool PAGED, bool APPEND>
-__global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(APPEND ? 1 : 2, APPEND ? 1 : 2))) void decode_mfma_flat(
+template <int D, int G, bool PAGED, bool APPEND, bool PAD>
+__global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(APPEND || PAD ? 1 : 2, APPEND || PAD ? 1 : 2))) void decode_mfma_flat(
     const DecodeArgs a) {
     static_assert(G == 4 || G == 8, "heads per workgroup");
     static_assert(D == 64 || D == 128, "head dims of the matrix-core decode kernel");
+    constexpr int kLimbs = q_limbs<PAD>();
+    constexpr int kQBits = 8 * kLimbs - 2;
     constexpr int NJ = D / 64;
     constexpr int NB = D / 16;
     constexpr int RPLV = kWave / NB;
@@ -678,7 +737,10 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
     const int unit = blockIdx.x - item * U;
     const int kvh = unit / a.nsg;
     const int sgi = unit - kvh * a.nsg;
-    const int hq0 = kvh * a.G + sgi * G;
+    const int d = PAD ? a.d : D;
+    const int sgh = PAD ? a.sgh : G;
+    const int hc = PAD ? min(sgh, a.G - sgi * sgh) : G;
+    const int hq0 = kvh * a.G + sgi * sgh;
     const int Wn = a.fit_items * kMWaves;
     const int wv = __builtin_amdgcn_readfirstlane(wave);
     const int gw = item * kMWaves + wv;
@@ -814,22 +876,23 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
             while (empty) {
                 const int be = c0 + __builtin_ctzll(empty);
                 empty &= empty - 1;
-                for (int i = lane; i < G * D; i += kWave) a.out[(static_cast<size_t>(be) * a.Hq + hq0) * D + i] = 0.0f;
+                for (int i = lane; i < hc * d; i += kWave) a.out[(static_cast<size_t>(be) * a.Hq + hq0) * d + i] = 0.0f;
             }
         }
     }
 
     constexpr bool app = APPEND;  // a.k_new != nullptr
     // q of head (r % G) of sequence b, dims 16g.. of each 64-dim block.
-    const int hrow = r % G;
+    const int hrow = PAD ? min(r % G, hc - 1) : r % G;
     float qv[16 * NJ];
     auto load_q = [&](int b) {
-        const float* qp = a.q + (static_cast<size_t>(b) * a.Hq + hq0 + hrow) * D + 16 * g;
+        const float* qp = a.q + (static_cast<size_t>(b) * a.Hq + hq0 + hrow) * d + 16 * g;
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
 #pragma unroll
             for (int i4 = 0; i4 < 4; i4++) {
-                const float4 x = *reinterpret_cast<const float4*>(qp + 64 * j + 4 * i4);
+                const float4 x = !PAD || 64 * j + 16 * g < d ? *reinterpret_cast<const float4*>(qp + 64 * j + 4 * i4)
+                                                             : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                 qv[16 * j + 4 * i4] = x.x;
                 qv[16 * j + 4 * i4 + 1] = x.y;
                 qv[16 * j + 4 * i4 + 2] = x.z;
@@ -837,7 +900,7 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
             }
         }
     };
-    i32x4 qb[NJ][3];
+    i32x4 qb[NJ][kLimbs];
     float qs = 0.0f;
     auto prepare_q = [&]() {
         float qmax = 0.0f;
@@ -847,23 +910,23 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
         qmax = fmaxf(qmax, __shfl_xor(qmax, 32));
         int qexp = 0;
         frexpf(qmax, &qexp);
-        const int E = qmax > 0.0f ? min(max(22 - qexp, -100), 126) : 0;
+        const int E = qmax > 0.0f ? min(max(kQBits - qexp, -100), 126) : 0;
         qs = ldexpf(1.0f, -E) * a.scale_log2;
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
-            int limb[3][16];
+            int limb[kLimbs][16];
 #pragma unroll
             for (int i = 0; i < 16; i++) {
-                const int Q = static_cast<int>(__builtin_rintf(ldexpf(qv[16 * j + i], E)));
-                const int l2 = ((Q + 128) & 255) - 128;
-                const int Q1 = (Q - l2) >> 8;
-                const int l1 = ((Q1 + 128) & 255) - 128;
-                limb[0][i] = (Q1 - l1) >> 8;
-                limb[1][i] = l1;
-                limb[2][i] = l2;
+                int Q = static_cast<int>(__builtin_rintf(ldexpf(qv[16 * j + i], E)));
+#pragma unroll
+                for (int lb = kLimbs - 1; lb > 0; lb--) {
+                    limb[lb][i] = ((Q + 128) & 255) - 128;
+                    Q = (Q - limb[lb][i]) >> 8;
+                }
+                limb[0][i] = Q;
             }
 #pragma unroll
-            for (int lb = 0; lb < 3; lb++)
+            for (int lb = 0; lb < kLimbs; lb++)
                 qb[j][lb] = i32x4{pack_bytes(&limb[lb][0]), pack_bytes(&limb[lb][4]), pack_bytes(&limb[lb][8]),
                                   pack_bytes(&limb[lb][12])};
         }
@@ -887,6 +950,14 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
     const int kvo = r * D + 16 * g;
     const int vvo = (lane / NB) * D + 16 * (lane % NB);
     const int svo = 16 * g;
+    auto k_off = [&](int s, int j) {
+        if constexpr (!PAD) return kvo + s * 16 * D + 64 * j;
+        else return 64 * j + 16 * g < d ? (r + 16 * s) * d + 16 * g + 64 * j : kOobOffset;
+    };
+    auto v_off = [&](int c) {
+        if constexpr (!PAD) return vvo + c * RPLV * D;
+        else return 16 * (lane % NB) < d ? (lane / NB + c * RPLV) * d + 16 * (lane % NB) : kOobOffset;
+    };
     // Tile loads of sequence b at token `base` (a multiple of 32).  `none`:
     // past the wave's range -- the same loads through empty resources (they
     // read zeros and touch no memory), so that every iteration issues the
@@ -898,8 +969,8 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
     auto set_load_seq = [&](int b) {
         if constexpr (!PAGED) {
             const size_t row0 = (static_cast<size_t>(b) * a.Hkv + kvh) * a.cap;
-            lkr = make_rsrc(a.k + row0 * D, cap * D);
-            lvr = make_rsrc(a.v + row0 * D, cap * D);
+            lkr = make_rsrc(a.k + row0 * d, cap * d);
+            lvr = make_rsrc(a.v + row0 * d, cap * d);
             lksr = make_rsrc(a.ks + row0, cap * 4u);
             lvsr = make_rsrc(a.vs + row0, cap * 4u);
         }
@@ -930,8 +1001,8 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
             pf_page = table_load(b, pf_base);
             const size_t rp = (static_cast<size_t>(page) * a.Hkv + kvh) * a.pages.size + (base & (a.pages.size - 1));
             const unsigned rem = static_cast<unsigned>(a.pages.size - (base & (a.pages.size - 1)));
-            kr = make_rsrc(a.k + rp * D, rem * D);
-            vr = make_rsrc(a.v + rp * D, rem * D);
+            kr = make_rsrc(a.k + rp * d, rem * d);
+            vr = make_rsrc(a.v + rp * d, rem * d);
             ksr = make_rsrc(a.ks + rp, rem * 4u);
             vsr = make_rsrc(a.vs + rp, rem * 4u);
             ko = so = 0;
@@ -940,17 +1011,17 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
             vr = lvr;
             ksr = lksr;
             vsr = lvsr;
-            ko = base * D;
+            ko = base * d;
             so = base * 4;
         }
 #pragma unroll
         for (int s = 0; s < 2; s++) {
 #pragma unroll
-            for (int j = 0; j < NJ; j++) Tt.ka[s][j] = buffer_load16_stream(kr, kvo + s * 16 * D + 64 * j, ko);
+            for (int j = 0; j < NJ; j++) Tt.ka[s][j] = buffer_load16_stream(kr, k_off(s, j), ko);
         }
 #pragma unroll
         for (int c = 0; c < NV; c++) {
-            const v4i_t x = buffer_load16_stream(vr, vvo + c * RPLV * D, ko);
+            const v4i_t x = buffer_load16_stream(vr, v_off(c), ko);
             Tt.v[c] = make_int4(x.x, x.y, x.z, x.w);
         }
 #pragma unroll
@@ -984,14 +1055,16 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
     float newks = 0.0f, newvs = 0.0f;
     auto load_new = [&](int b) {
         const size_t bh = static_cast<size_t>(b) * a.Hkv + kvh;
+        auto elem = [&](int j) {
+            const int e = (lane + kWave * j) & (D - 1);
+            return !PAD || e < d ? (j < NJ ? a.k_new : a.v_new)[bh * d + e] : 0.0f;
+        };
         if (x_issue & 1) {
 #pragma unroll
-            for (int j = 0; j < NE; j++)
-                xnew1[j] = (j < NJ ? a.k_new : a.v_new)[bh * D + ((lane + kWave * j) & (D - 1))];
+            for (int j = 0; j < NE; j++) xnew1[j] = elem(j);
         } else {
 #pragma unroll
-            for (int j = 0; j < NE; j++)
-                xnew0[j] = (j < NJ ? a.k_new : a.v_new)[bh * D + ((lane + kWave * j) & (D - 1))];
+            for (int j = 0; j < NE; j++) xnew0[j] = elem(j);
         }
         x_issue++;
     };
@@ -1016,8 +1089,9 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
         if (sgi == 0) {
             if (lane < 2 * NB) {
                 const int row = lane / NB, piece = lane % NB;
-                *reinterpret_cast<int4*>((row ? a.v : a.k) + rnew * D + 16 * piece) =
-                    *reinterpret_cast<const int4*>(&s_newq[wv][row][16 * piece]);
+                if (!PAD || 16 * piece < d)
+                    *reinterpret_cast<int4*>((row ? a.v : a.k) + rnew * d + 16 * piece) =
+                        *reinterpret_cast<const int4*>(&s_newq[wv][row][16 * piece]);
             }
             if (lane == 0) {
                 a.ks[rnew] = newks;
@@ -1048,11 +1122,11 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
 
     // One tile of the current sequence (tokens [base, base + 32) of len).
     auto compute = [&](const Tile& Tt, int base, int len, const int8_t* vt) {
-        i32x4 cq[2][3];
+        i32x4 cq[2][kLimbs];
 #pragma unroll
         for (int s = 0; s < 2; s++) {
 #pragma unroll
-            for (int lb = 0; lb < 3; lb++) {
+            for (int lb = 0; lb < kLimbs; lb++) {
                 i32x4 c = i32x4{0, 0, 0, 0};
 #pragma unroll
                 for (int j = 0; j < NJ; j++) c = __builtin_amdgcn_mfma_i32_16x16x64_i8(Tt.ka[s][j], qb[j][lb], c, 0, 0, 0);
@@ -1065,8 +1139,9 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
         for (int s = 0; s < 2; s++) {
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const int low = (cq[s][1][i] << 8) + cq[s][2][i];
-                const float dot = static_cast<float>(cq[s][0][i]) * 65536.0f + static_cast<float>(low);
+                const int low = (cq[s][kLimbs - 2][i] << 8) + cq[s][kLimbs - 1][i];
+                const int high = kLimbs == 4 ? (cq[s][0][i] << 8) + cq[s][1][i] : cq[s][0][i];
+                const float dot = fmaf(static_cast<float>(high), 65536.0f, static_cast<float>(low));
                 sc[4 * s + i] = (dot * Tt.ks[s][i]) * qs;
                 vsv[4 * s + i] = Tt.vs[s][i];
             }
@@ -1094,8 +1169,8 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
         const float mn = fmaxf(m, mt);
         const float ms = mn == -INFINITY ? 0.0f : mn;
         const float alpha = fast_exp2(m - ms);
-        const float vn = fmaxf(vref, vmax);
-        const float rvn = vn > 0.0f ? __builtin_amdgcn_rcpf(vn) : 0.0f;
+        const float vn = fmaxf(vref, PAD ? pow2_above(vmax) : vmax);
+        const float rvn = vn > 0.0f ? __builtin_amdgcn_rcpf(vn) : 0.0f;  // v_rcp_f32, 1 ulp (PAD: exact)
         const float f = vn > 0.0f ? alpha * (vref * rvn) : alpha;
         const float winv = kPScale * rvn;
         m = mn;
@@ -1131,11 +1206,11 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
         lt += __shfl_xor(lt, 16);
         lt += __shfl_xor(lt, 32);
         const float fct = vref * (1.0f / kPScale);
-        const bool writer = r < G;
+        const bool writer = r < hc;
         const size_t row = static_cast<size_t>(b) * a.Hq + hq0 + r;
         const size_t rec = (static_cast<size_t>(gw) + b) * a.Hq + hq0 + r;
         const float sc = complete ? fct / lt : fct;
-        const buf_rsrc recr = make_rsrc(a.part_acc + (static_cast<size_t>(gw) + b) * a.Hq * D, a.Hq * D * 4u);
+        const buf_rsrc recr = make_rsrc(a.part_acc + (static_cast<size_t>(gw) + b) * a.Hq * d, a.Hq * d * 4u);
 #pragma unroll
         for (int c = 0; c < NB; c++) {
             f32x4 o;
@@ -1144,14 +1219,14 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
             for (int i = 0; i < 4; i++)
                 o[i] = (acc[c][i] + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc[c][i]),
                                                                                  0x100 + G, 0xF, 0xF, false))) * sc;
-            if (writer) {
+            if (writer && (!PAD || 16 * c < d)) {
                 if (complete) {
 #pragma unroll
-                    for (int i = 0; i < 4; i++) a.out[row * D + 16 * c + 4 * g + i] = o[i];
+                    for (int i = 0; i < 4; i++) a.out[row * d + 16 * c + 4 * g + i] = o[i];
                 } else {
                     // Device-coherent 16-byte store (sc1), as put_coherent.
                     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i_t, o), recr,
-                                                           ((hq0 + r) * D + 16 * c + 4 * g) * 4, 0, kCoherent);
+                                                           ((hq0 + r) * d + 16 * c + 4 * g) * 4, 0, kCoherent);
                 }
             }
         }
@@ -1320,7 +1395,7 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
         const int bn = k == 0 ? pm_n : cn;
         const int w0 = wave_of(bE, b);
         const int w1 = wave_of(bE + bn - 1, b);
-        merge_wave_records<D, G>(a, b, w0, w1 - w0 + 1, hq0, lane);
+        merge_wave_records<D, G, PAD>(a, b, w0, w1 - w0 + 1, hq0, hc, lane);
     }
 }
 
@@ -1328,41 +1403,48 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
 
 int mfma_tile_tokens() { return kMBStep; }
 
+// Heads per workgroup: G heads in ceil(G / 8) groups as equal as they come.
 int mfma_heads_per_group(int G, int d) {
-    if (d != 64 && d != 128) return 0;
-    if (G % 8 == 0) return 8;
-    if (G % 4 == 0) return 4;
-    return 0;
+    if (G < 2 || d % 16 != 0 || d < 48 || d > 128) return 0;
+    const int groups = (G + 7) / 8;
+    return (G + groups - 1) / groups;
 }
 
 namespace {
-template <int D, int G>
+template <int D, int G, bool PAD>
 void launch_mfma_dg(const DecodeArgs& a, dim3 grid, dim3 block, hipStream_t stream) {
     const bool paged = a.pages.table != nullptr;
     if (a.flat) {
         const bool app = a.k_new != nullptr;
-        if (paged && app) hipLaunchKernelGGL((decode_mfma_flat<D, G, true, true>), grid, block, 0, stream, a);
-        else if (paged) hipLaunchKernelGGL((decode_mfma_flat<D, G, true, false>), grid, block, 0, stream, a);
-        else if (app) hipLaunchKernelGGL((decode_mfma_flat<D, G, false, true>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((decode_mfma_flat<D, G, false, false>), grid, block, 0, stream, a);
+        if (paged && app) hipLaunchKernelGGL((decode_mfma_flat<D, G, true, true, PAD>), grid, block, 0, stream, a);
+        else if (paged) hipLaunchKernelGGL((decode_mfma_flat<D, G, true, false, PAD>), grid, block, 0, stream, a);
+        else if (app) hipLaunchKernelGGL((decode_mfma_flat<D, G, false, true, PAD>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((decode_mfma_flat<D, G, false, false, PAD>), grid, block, 0, stream, a);
     } else if (a.fit_items > 0) {
-        if (paged) hipLaunchKernelGGL((decode_mfma<D, G, true, true>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((decode_mfma<D, G, false, true>), grid, block, 0, stream, a);
+        if (paged) hipLaunchKernelGGL((decode_mfma<D, G, true, true, PAD>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((decode_mfma<D, G, false, true, PAD>), grid, block, 0, stream, a);
     } else {
-        if (paged) hipLaunchKernelGGL((decode_mfma<D, G, true, false>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((decode_mfma<D, G, false, false>), grid, block, 0, stream, a);
+        if (paged) hipLaunchKernelGGL((decode_mfma<D, G, true, false, PAD>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((decode_mfma<D, G, false, false, PAD>), grid, block, 0, stream, a);
     }
+}
+template <int D, int G>
+void launch_mfma_pad(const DecodeArgs& a, dim3 grid, dim3 block, hipStream_t stream) {
+    if (a.d != D || a.sgh != G || a.G % G != 0) launch_mfma_dg<D, G, true>(a, grid, block, stream);
+    else launch_mfma_dg<D, G, false>(a, grid, block, stream);
 }
 }  // namespace
 
-hipError_t launch_decode_mfma(const DecodeArgs& a, const DecodePlan& p, hipStream_t stream) {
-    const dim3 grid(static_cast<unsigned>(decode_grid(a, p)));
+hipError_t launch_decode_mfma(const DecodeArgs& a0, const DecodePlan& p, hipStream_t stream) {
+    const dim3 grid(static_cast<unsigned>(decode_grid(a0, p)));
     const dim3 block(kMWaves * kWave);
-    if (a.d == 128 && p.sg == 4) launch_mfma_dg<128, 4>(a, grid, block, stream);
-    else if (a.d == 128 && p.sg == 8) launch_mfma_dg<128, 8>(a, grid, block, stream);
-    else if (a.d == 64 && p.sg == 4) launch_mfma_dg<64, 4>(a, grid, block, stream);
-    else if (a.d == 64 && p.sg == 8) launch_mfma_dg<64, 8>(a, grid, block, stream);
-    else return hipErrorInvalidValue;
+    if (p.sg < 1 || p.sg > 8 || a0.d > 128 || a0.d % 16 != 0) return hipErrorInvalidValue;
+    DecodeArgs a = a0;
+    a.sgh = p.sg;
+    if (a.d > 64 && p.sg <= 4) launch_mfma_pad<128, 4>(a, grid, block, stream);
+    else if (a.d > 64) launch_mfma_pad<128, 8>(a, grid, block, stream);
+    else if (p.sg <= 4) launch_mfma_pad<64, 4>(a, grid, block, stream);
+    else launch_mfma_pad<64, 8>(a, grid, block, stream);
     return hipGetLastError();
 }
 

@@ -55,7 +55,8 @@ struct DecodeArgs {
     int max_len;             // every length is clamped to [0, max_len], max_len <= cap
     int splits;              // grid splits per sequence (static splits)
     int chunk;               // tokens per split (static splits)
-    int nsg;                 // head groups per kv head (G / heads per workgroup)
+    int nsg;                 // head groups per kv head (G / heads per workgroup, rounded up)
+    int sgh;                 // heads per workgroup (matrix-core kernel)
     int lpt_target;          // > 0: the matrix-core kernel derives the split schedule itself (locate_lpt)
                              // for this many workgroups per round (the schedule kernel's target) ...
     int lpt_target_log2;     // ... a power of two, 2^lpt_target_log2
@@ -111,7 +112,7 @@ constexpr int kSizeClasses = 64;
 enum class Kernel {
     Generic,  // any head dim / alignment (decode_generic)
     Valu,     // decode_fast: d in {32,64,128,256}, per-lane FMAs
-    Mfma,     // decode_mfma: d = 128, 4 or 8 query heads per kv head group
+    Mfma,     // decode_mfma: d a multiple of 16 up to 128, up to 8 query heads per kv head group
 };
 
 // Launch plan chosen on the host.
@@ -120,7 +121,7 @@ struct DecodePlan {
     bool fast;       // a tuned kernel (Valu or Mfma): 16-byte aligned rows
     int sg;          // query heads per workgroup (tuned kernels)
     int tile;        // tokens one workgroup iteration covers (tuned kernels; 0: generic)
-    int nsg;         // G / sg
+    int nsg;         // G / sg, rounded up
     int splits;      // splits per sequence (grid dimension)
     int chunk;       // tokens per split
     bool counters;   // last-arriving split merges (fast path with a zeroed counter prefix)
