@@ -1430,7 +1430,11 @@ void launch_mfma_dg(const DecodeArgs& a, dim3 grid, dim3 block, hipStream_t stre
 }
 template <int D, int G>
 void launch_mfma_pad(const DecodeArgs& a, dim3 grid, dim3 block, hipStream_t stream) {
-    if (a.d != D || a.sgh != G || a.G % G != 0) launch_mfma_dg<D, G, true>(a, grid, block, stream);
+    // Rows whose scale quads are not 16-byte aligned run on PAD instances for
+    // their four q limbs (they ran on the fp32 FMA kernel before).
+    const uintptr_t scales = reinterpret_cast<uintptr_t>(a.ks) | reinterpret_cast<uintptr_t>(a.vs);
+    const bool odd = (scales & 15u) != 0 || (a.pages.table == nullptr && a.cap % 4 != 0);
+    if (a.d != D || a.sgh != G || a.G % G != 0 || odd) launch_mfma_dg<D, G, true>(a, grid, block, stream);
     else launch_mfma_dg<D, G, false>(a, grid, block, stream);
 }
 }  // namespace
