@@ -212,7 +212,7 @@ DecodePlan make_plan(int B, int Hq, int Hkv, int d, int max_len, bool aligned, b
     const bool pow2 = page > 0 && (page & (page - 1)) == 0;
     const int wave_tokens = kvq::fast_wave_tokens(d, sg_v);
     const bool valu_pages = page == 0 || (pow2 && wave_tokens > 0 && page % wave_tokens == 0);
-    const bool mfma_pages = page == 0 || (pow2 && page % 32 == 0 && page < (1 << 24));
+    const bool mfma_pages = page == 0 || (pow2 && page >= 16 && page < (1 << 24));
     int tile = 0;
     const int force = forced_kernel();
     if (force == kForceGeneric) aligned = false;

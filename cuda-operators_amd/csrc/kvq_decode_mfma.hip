@@ -127,7 +127,20 @@ constexpr int q_limbs() { return PAD ? 4 : 3; }
 // heads 171 / 43 us, 12 heads (two groups of 6) 95 / 68 us; B64 2 heads L
 // 300-4K 99 / 69 us; B8 3 heads d96 L 500-3K 1417 / 20 us.
 
-template <int D, int G, bool PAGED, bool FIT, bool PAD>
+// PAGED: 0 contiguous, 1 pages of 32 tokens or more (a tile lies in one page),
+// 2 pages of 16 (PAD only).  Buffer resources of kv head kvh's rows in one
+// 16-token page.
+__device__ __forceinline__ void page16_rsrc(const DecodeArgs& a, int kvh, int id, int d, buf_rsrc& kr, buf_rsrc& vr,
+                                            buf_rsrc& ksr, buf_rsrc& vsr) {
+    const int page = min(max(__builtin_amdgcn_readfirstlane(id), 0), a.pages.num_pages - 1);
+    const size_t rp = (static_cast<size_t>(page) * a.Hkv + kvh) * 16;
+    kr = make_rsrc(a.k + rp * d, 16 * d);
+    vr = make_rsrc(a.v + rp * d, 16 * d);
+    ksr = make_rsrc(a.ks + rp, 64u);
+    vsr = make_rsrc(a.vs + rp, 64u);
+}
+
+template <int D, int G, int PAGED, bool FIT, bool PAD>
 __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(2))) void decode_mfma(
     const DecodeArgs a) {
     static_assert(G == 4 || G == 8, "heads per workgroup");
@@ -344,6 +357,13 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
         if constexpr (!PAD) return vvo + c * RPLV * D;
         else return 16 * (lane % NB) < d ? (lane / NB + c * RPLV) * d + 16 * (lane % NB) : kOobOffset;
     };
+    // PAGED 2 (16-token pages): a tile is two pages, sub-tile s of K and the
+    // scales in page s, V load c in page c * RPLV / 16.  The two ids come in
+    // one 8-byte load (the second reads 0 past the table's row).  These pages
+    // ran on the FMA kernel, whose wave tile is 16 tokens: B32 Hq32/Hkv8 d128
+    // L 200-4000 with append 76.5 us (a schedule launch of 7.5 us among it),
+    // here 43.4 us; 7 heads per kv head 169 / 46 us; d = 64 (a 32-token wave
+    // tile there, so the generic kernel) B4 L 3000 1079 / 9.9 us.
     // Paged: each tile's page id comes from the block table one tile ahead,
     // by a vector load issued before the previous tile's K/V loads, so a
     // tile's loads wait only for that id (in-order vector-memory counter),
@@ -356,19 +376,27 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
                   PAGED ? static_cast<unsigned>(a.pages.max_pages) * 4u : 0u);
     auto fetch_page = [&](int it) {
         const int pi = min((wbase + it * kMBStep) >> a.pages.shift, a.pages.max_pages - 1);
-        return __builtin_amdgcn_raw_buffer_load_b32(tabr, pi * 4, 0, 0);
+        if constexpr (PAGED == 2) return __builtin_bit_cast(i32x2, __builtin_amdgcn_raw_buffer_load_b64(tabr, pi * 4, 0, 0));
+        else return i32x2{buffer_load4(tabr, pi * 4, 0), 0};
     };
-    int pg_next = 0;
+    i32x2 pg_next = {0, 0};
     if constexpr (PAGED) pg_next = fetch_page(0);
     auto load_tile = [&](Tile& T, int it) {
         const int base = wbase + it * kMBStep;
         int ko = base * d;
         int so = base * 4;
         buf_rsrc kr = kres, vr = vres, ksr = ksres, vsr = vsres;
-        if constexpr (PAGED) {
+        buf_rsrc kr1 = kr, vr1 = vr, ksr1 = ksr, vsr1 = vsr;
+        if constexpr (PAGED == 2) {
+            const i32x2 id = pg_next;
+            pg_next = fetch_page(it + 1);
+            page16_rsrc(a, kvh, id.x, d, kr, vr, ksr, vsr);
+            page16_rsrc(a, kvh, id.y, d, kr1, vr1, ksr1, vsr1);
+            ko = so = 0;
+        } else if constexpr (PAGED == 1) {
             // The tile lies in one page (page size a multiple of 32): resources
             // from its first token to the end of that page.
-            const int page = min(max(__builtin_amdgcn_readfirstlane(pg_next), 0), a.pages.num_pages - 1);
+            const int page = min(max(__builtin_amdgcn_readfirstlane(pg_next.x), 0), a.pages.num_pages - 1);
             pg_next = fetch_page(it + 1);
             const size_t rp = (static_cast<size_t>(page) * a.Hkv + kvh) * a.pages.size + (base & (a.pages.size - 1));
             const unsigned rem = static_cast<unsigned>(a.pages.size - (base & (a.pages.size - 1)));
@@ -381,17 +409,20 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
         for (int s = 0; s < 2; s++) {
 #pragma unroll
-            for (int j = 0; j < NJ; j++) T.ka[s][j] = buffer_load16_stream(kr, k_off(s, j), ko);
+            for (int j = 0; j < NJ; j++)
+                T.ka[s][j] = PAGED == 2 ? buffer_load16_stream(s ? kr1 : kr, k_off(0, j), 0)
+                                        : buffer_load16_stream(kr, k_off(s, j), ko);
         }
 #pragma unroll
         for (int c = 0; c < NV; c++) {
-            const v4i_t x = buffer_load16_stream(vr, v_off(c), ko);
+            const v4i_t x = PAGED == 2 ? buffer_load16_stream(c * RPLV >= 16 ? vr1 : vr, v_off(c % (16 / RPLV)), 0)
+                                       : buffer_load16_stream(vr, v_off(c), ko);
             T.v[c] = make_int4(x.x, x.y, x.z, x.w);
         }
 #pragma unroll
         for (int s = 0; s < 2; s++) {
-            const v4i_t xk = buffer_load16(ksr, svo + 64 * s, so);
-            const v4i_t xv = buffer_load16(vsr, svo + 64 * s, so);
+            const v4i_t xk = PAGED == 2 ? buffer_load16(s ? ksr1 : ksr, svo, 0) : buffer_load16(ksr, svo + 64 * s, so);
+            const v4i_t xv = PAGED == 2 ? buffer_load16(s ? vsr1 : vsr, svo, 0) : buffer_load16(vsr, svo + 64 * s, so);
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 T.ks[s][i] = __int_as_float(xk[i]);
@@ -709,7 +740,7 @@ __device__ inline void merge_wave_records(const DecodeArgs& a, int b, int w0, in
     }
 }
 
-template <int D, int G, bool PAGED, bool APPEND, bool PAD>
+template <int D, int G, int PAGED, bool APPEND, bool PAD>
 __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(APPEND || PAD ? 1 : 2, APPEND || PAD ? 1 : 2))) void decode_mfma_flat(
     const DecodeArgs a) {
     static_assert(G == 4 || G == 8, "heads per workgroup");
@@ -980,31 +1011,39 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
     // waiting for it leaves them in flight) and used when that tile loads; a
     // move to another sequence looks its first page up at once.  Page sizes
     // are powers of two here; indices past a row are clamped into it.
-    int pf_b = -1, pf_base = 0, pf_page = 0;
+    int pf_b = -1, pf_base = 0;
+    i32x2 pf_page = {0, 0};
     auto table_load = [&](int b, int base) {
         const buf_rsrc tabr = make_rsrc(a.pages.table + static_cast<size_t>(b) * a.pages.max_pages,
                                         static_cast<unsigned>(a.pages.max_pages) * 4u);
-        return __builtin_amdgcn_raw_buffer_load_b32(tabr, min(base >> a.pages.shift, a.pages.max_pages - 1) * 4, 0, 0);
+        const int pi = min(base >> a.pages.shift, a.pages.max_pages - 1);
+        if constexpr (PAGED == 2) return __builtin_bit_cast(i32x2, __builtin_amdgcn_raw_buffer_load_b64(tabr, pi * 4, 0, 0));
+        else return i32x2{buffer_load4(tabr, pi * 4, 0), 0};
     };
     auto load_tile = [&](Tile& Tt, int b, int base, bool none) {
-        buf_rsrc kr, vr, ksr, vsr;
+        buf_rsrc kr, vr, ksr, vsr, kr1, vr1, ksr1, vsr1;
         int ko, so;
         if (none) {
-            kr = vr = ksr = vsr = make_rsrc(a.k, 0u);
+            kr = vr = ksr = vsr = kr1 = vr1 = ksr1 = vsr1 = make_rsrc(a.k, 0u);
             ko = so = 0;
         } else if constexpr (PAGED) {
-            int id = pf_page;
+            i32x2 id = pf_page;
             if (b != pf_b || base != pf_base) id = table_load(b, base);
-            const int page = min(max(__builtin_amdgcn_readfirstlane(id), 0), a.pages.num_pages - 1);
             pf_b = b;
             pf_base = base + kMTile;
             pf_page = table_load(b, pf_base);
-            const size_t rp = (static_cast<size_t>(page) * a.Hkv + kvh) * a.pages.size + (base & (a.pages.size - 1));
-            const unsigned rem = static_cast<unsigned>(a.pages.size - (base & (a.pages.size - 1)));
-            kr = make_rsrc(a.k + rp * d, rem * d);
-            vr = make_rsrc(a.v + rp * d, rem * d);
-            ksr = make_rsrc(a.ks + rp, rem * 4u);
-            vsr = make_rsrc(a.vs + rp, rem * 4u);
+            if constexpr (PAGED == 2) {
+                page16_rsrc(a, kvh, id.x, d, kr, vr, ksr, vsr);
+                page16_rsrc(a, kvh, id.y, d, kr1, vr1, ksr1, vsr1);
+            } else {
+                const int page = min(max(__builtin_amdgcn_readfirstlane(id.x), 0), a.pages.num_pages - 1);
+                const size_t rp = (static_cast<size_t>(page) * a.Hkv + kvh) * a.pages.size + (base & (a.pages.size - 1));
+                const unsigned rem = static_cast<unsigned>(a.pages.size - (base & (a.pages.size - 1)));
+                kr = make_rsrc(a.k + rp * d, rem * d);
+                vr = make_rsrc(a.v + rp * d, rem * d);
+                ksr = make_rsrc(a.ks + rp, rem * 4u);
+                vsr = make_rsrc(a.vs + rp, rem * 4u);
+            }
             ko = so = 0;
         } else {
             kr = lkr;
@@ -1017,17 +1056,20 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
         for (int s = 0; s < 2; s++) {
 #pragma unroll
-            for (int j = 0; j < NJ; j++) Tt.ka[s][j] = buffer_load16_stream(kr, k_off(s, j), ko);
+            for (int j = 0; j < NJ; j++)
+                Tt.ka[s][j] = PAGED == 2 ? buffer_load16_stream(s ? kr1 : kr, k_off(0, j), 0)
+                                         : buffer_load16_stream(kr, k_off(s, j), ko);
         }
 #pragma unroll
         for (int c = 0; c < NV; c++) {
-            const v4i_t x = buffer_load16_stream(vr, v_off(c), ko);
+            const v4i_t x = PAGED == 2 ? buffer_load16_stream(c * RPLV >= 16 ? vr1 : vr, v_off(c % (16 / RPLV)), 0)
+                                       : buffer_load16_stream(vr, v_off(c), ko);
             Tt.v[c] = make_int4(x.x, x.y, x.z, x.w);
         }
 #pragma unroll
         for (int s = 0; s < 2; s++) {
-            const v4i_t xk = buffer_load16(ksr, svo + 64 * s, so);
-            const v4i_t xv = buffer_load16(vsr, svo + 64 * s, so);
+            const v4i_t xk = PAGED == 2 ? buffer_load16(s ? ksr1 : ksr, svo, 0) : buffer_load16(ksr, svo + 64 * s, so);
+            const v4i_t xv = PAGED == 2 ? buffer_load16(s ? vsr1 : vsr, svo, 0) : buffer_load16(vsr, svo + 64 * s, so);
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 Tt.ks[s][i] = __int_as_float(xk[i]);
@@ -1411,31 +1453,28 @@ int mfma_heads_per_group(int G, int d) {
 }
 
 namespace {
-template <int D, int G, bool PAD>
+template <int D, int G, int PAGED, bool PAD>
 void launch_mfma_dg(const DecodeArgs& a, dim3 grid, dim3 block, hipStream_t stream) {
-    const bool paged = a.pages.table != nullptr;
     if (a.flat) {
-        const bool app = a.k_new != nullptr;
-        if (paged && app) hipLaunchKernelGGL((decode_mfma_flat<D, G, true, true, PAD>), grid, block, 0, stream, a);
-        else if (paged) hipLaunchKernelGGL((decode_mfma_flat<D, G, true, false, PAD>), grid, block, 0, stream, a);
-        else if (app) hipLaunchKernelGGL((decode_mfma_flat<D, G, false, true, PAD>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((decode_mfma_flat<D, G, false, false, PAD>), grid, block, 0, stream, a);
+        if (a.k_new) hipLaunchKernelGGL((decode_mfma_flat<D, G, PAGED, true, PAD>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((decode_mfma_flat<D, G, PAGED, false, PAD>), grid, block, 0, stream, a);
     } else if (a.fit_items > 0) {
-        if (paged) hipLaunchKernelGGL((decode_mfma<D, G, true, true, PAD>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((decode_mfma<D, G, false, true, PAD>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((decode_mfma<D, G, PAGED, true, PAD>), grid, block, 0, stream, a);
     } else {
-        if (paged) hipLaunchKernelGGL((decode_mfma<D, G, true, false, PAD>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((decode_mfma<D, G, false, false, PAD>), grid, block, 0, stream, a);
+        hipLaunchKernelGGL((decode_mfma<D, G, PAGED, false, PAD>), grid, block, 0, stream, a);
     }
 }
 template <int D, int G>
 void launch_mfma_pad(const DecodeArgs& a, dim3 grid, dim3 block, hipStream_t stream) {
-    // Rows whose scale quads are not 16-byte aligned run on PAD instances for
-    // their four q limbs (they ran on the fp32 FMA kernel before).
+    // Rows whose scale quads are not 16-byte aligned, and 16-token pages, run on
+    // PAD instances for their four q limbs (they ran on the fp32 FMA kernel before).
     const uintptr_t scales = reinterpret_cast<uintptr_t>(a.ks) | reinterpret_cast<uintptr_t>(a.vs);
     const bool odd = (scales & 15u) != 0 || (a.pages.table == nullptr && a.cap % 4 != 0);
-    if (a.d != D || a.sgh != G || a.G % G != 0 || odd) launch_mfma_dg<D, G, true>(a, grid, block, stream);
-    else launch_mfma_dg<D, G, false>(a, grid, block, stream);
+    const bool paged = a.pages.table != nullptr;
+    if (paged && a.pages.size < kMTile) launch_mfma_dg<D, G, 2, true>(a, grid, block, stream);
+    else if (a.d != D || a.sgh != G || a.G % G != 0 || odd)
+        paged ? launch_mfma_dg<D, G, 1, true>(a, grid, block, stream) : launch_mfma_dg<D, G, 0, true>(a, grid, block, stream);
+    else paged ? launch_mfma_dg<D, G, 1, false>(a, grid, block, stream) : launch_mfma_dg<D, G, 0, false>(a, grid, block, stream);
 }
 }  // namespace
 
