@@ -1,51 +1,25 @@
-// kvq_attention.hip -- dense fp32 attention forward on gfx950 matrix cores:
-// out = softmax(Q K^T / sqrt(d)) V for Q[M,d], K/V[N,d] (one head), the math
-// of the reference's attention_online_launch (attention/softmax_new.cu:87-281).
+// kvq_attention.hip -- dense fp32 attention forward on gfx950: out =
+// softmax(Q K^T / sqrt(d)) V for Q[M,d], K/V[N,d] (one head), the math of the
+// reference's attention_online_launch (attention/softmax_new.cu:87-281).
 //
-// attention_mfma<D> (d in {32, 64, 128, 256}): a workgroup of 8 waves owns
-// 128 queries (16 per wave) and one split of the keys, which it streams
-// through LDS in 64-key tiles (32 at d = 256) shared by all its waves (two
-// LDS buffers: one barrier per tile; 135 KB of LDS at d = 128).  Both products run on
-// v_mfma_f32_16x16x4_f32 (fp32 in, fp32 accumulate: the same arithmetic as
-// fp32 FMAs, in another order):
-//   * S^T = K Q^T per 16-key block: A = K rows from LDS, B = this wave's q
-//     (held in registers, pre-scaled by softmax_scale * log2 e); the k index
-//     g = lane / 16 of step s is dim g * D/4 + s, so each lane reads its K
-//     operands as contiguous 16-byte LDS loads.  C leaves lane l with keys
-//     4g + i of query l % 16.
-//   * online softmax per query: max and sum over the lane's 16 keys of the
-//     tile and across the 4 lane groups (shuffles); exp2 of log2-unit scores.
-//   * O^T += V^T P^T: the P values stay in the registers the QK product left
-//     them in -- step i of a key block takes register i of every lane, i.e.
-//     keys {4g + i}, and the A operand reads V rows 4g + i to match.  Output
-//     rows (dims) of block c are dims (D/16) * m + c, so each lane's V
-//     operands are contiguous too.
+// Here: the kernels for few queries (attention_rows, attention_direct), the
+// merge of split records, and attention_generic (any d <= 1024 and any
+// alignment, one wave per query row).  The rest runs on attention_limbs
+// (kvq_attention_limbs.hpp).
+//
 // Keys are split over the grid's second dimension when the query blocks alone
 // cannot fill the GPU; splits write partial (m, l, acc) records and a second
 // launch, attention_merge, combines them over the whole grid (a merge by the
 // last split to arrive would leave the records of a query block to one CU,
 // whose far reads then dominate the launch).
-//
-// attention_generic: any d <= 1024 (one wave per query row, VALU), the
-// correctness path for other head dims.
 #include <math.h>
 
-#include "kvq_device.hpp"
-#include "kvq_internal.hpp"
+#include "kvq_attention.hpp"
+#include "kvq_attention_limbs.hpp"
 
 namespace kvq {
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// Waves per workgroup (16 queries each): kAttnBlockWide / 16, or
-// kAttnBlockNarrow / 16 when the wide blocks cannot fill the GPU.
-// Keys per LDS tile: 64, or 32 at d = 256 (two double-buffered K/V tiles of
-// 64 x 256 floats would not fit in LDS).
-template <int D>
-constexpr int attention_tile() {
-    return D >= 256 ? 32 : 64;
-}
 constexpr int kAttnMaxSplits = 1024;    // key splits per launch (the merge loops over them)
 
 // Merge of the split records: a group of 2^glog lanes (within one wave) per
@@ -58,7 +32,7 @@ constexpr int kAttnMaxSplits = 1024;    // key splits per launch (the merge loop
 constexpr int kMergeThreads = 256;
 template <int D>
 __global__ __launch_bounds__(kMergeThreads) void attention_merge(const AttnArgs a, int glog) {
-    constexpr int C4 = D / 4;
+    const int C4 = (D > 0 ? D : attention_record_dim(a.d)) / 4;
     const int G = 1 << glog;
     const int j = threadIdx.x & (G - 1);
     const int e = (blockIdx.x * kMergeThreads + threadIdx.x) >> glog;
@@ -124,201 +98,22 @@ __global__ __launch_bounds__(kMergeThreads) void attention_merge(const AttnArgs 
     }
     if (j == 0) {
         const float inv = 1.0f / L;
-        reinterpret_cast<float4*>(a.out)[e] = make_float4(A.x * inv, A.y * inv, A.z * inv, A.w * inv);
-    }
-}
-
-template <int D, int W>
-__global__ __launch_bounds__(W* kWave) void attention_mfma(const AttnArgs a) {
-    constexpr int DQ = D / 4;   // contraction dims per lane group in QK
-    constexpr int NB = D / 16;  // 16-dim output blocks; block c row m = dim NB * m + c
-    static_assert(NB % 4 == 0 || NB == 2, "V operand / output vector width");
-    constexpr int KS = D + 4;   // LDS row stride in floats (16-byte pad: conflict-free row reads)
-    constexpr int AK = attention_tile<D>();  // keys per tile
-    constexpr int KB = AK / 16;              // 16-key blocks per tile
-    constexpr int NL = AK * D / 4 / (W * kWave);  // float4 per thread per tile per tensor
-    static_assert(NL >= 1 && AK % 16 == 0, "tile load shape");
-    __shared__ __align__(16) float s_kv[2][2 * AK * KS];  // two (K tile, V tile) buffers
-    int cur = 0;
-
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wave = threadIdx.x / kWave;
-    const int r = lane & 15;
-    const int g = lane >> 4;
-    const int split = blockIdx.y;
-    const int q0 = blockIdx.x * (16 * W) + wave * 16;
-    const int k0 = split * a.chunk;
-    const int k1 = min(a.N, k0 + a.chunk);
-
-    // This wave's q^T operand: lane holds q[q0 + r][g * DQ + s], scaled.
-    float qv[DQ];
-    {
-        const float* qp = a.q + static_cast<size_t>(min(q0 + r, a.M - 1)) * D + g * DQ;
-#pragma unroll
-        for (int j = 0; j < DQ / 4; j++) {
-            const float4 x = *reinterpret_cast<const float4*>(qp + 4 * j);
-            qv[4 * j] = x.x * a.scale_log2;
-            qv[4 * j + 1] = x.y * a.scale_log2;
-            qv[4 * j + 2] = x.z * a.scale_log2;
-            qv[4 * j + 3] = x.w * a.scale_log2;
+        if (D > 0 || (a.d & 3) == 0) {
+            reinterpret_cast<float4*>(a.out)[e] = make_float4(A.x * inv, A.y * inv, A.z * inv, A.w * inv);
+        } else {
+            const int c = 4 * (e - q * C4);
+            float* const op = a.out + static_cast<size_t>(q) * a.d + c;
+            op[0] = A.x * inv;
+            if (c + 1 < a.d) op[1] = A.y * inv;
+            if (c + 2 < a.d) op[2] = A.z * inv;
+            if (c + 3 < a.d) op[3] = A.w * inv;
         }
-    }
-    f32x4 o[NB];
-#pragma unroll
-    for (int c = 0; c < NB; c++) o[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float m = -INFINITY, l = 0.0f;
-
-    // Tile loads: float4 f = threadIdx.x + j * (64 W) of the AK x D tile.
-    float4 pk[NL], pv[NL];
-    auto load_tile = [&](int t0) {
-#pragma unroll
-        for (int j = 0; j < NL; j++) {
-            const int f = threadIdx.x + j * W * kWave;
-            const int row = f / (D / 4);
-            const int c4 = f - row * (D / 4);
-            const int key = t0 + row;
-            // Rows past the split's end read its last row (in bounds) and are
-            // zeroed by a select.
-            const size_t kr = static_cast<size_t>(min(key, k1 - 1)) * D + 4 * c4;
-            const float keep = key < k1 ? 1.0f : 0.0f;
-            const float4 x = *reinterpret_cast<const float4*>(a.k + kr);
-            const float4 y = *reinterpret_cast<const float4*>(a.v + kr);
-            pk[j] = make_float4(x.x * keep, x.y * keep, x.z * keep, x.w * keep);
-            pv[j] = make_float4(y.x * keep, y.y * keep, y.z * keep, y.w * keep);
-        }
-    };
-    auto store_tile = [&](int buf) {
-        float* const s_k = s_kv[buf];
-        float* const s_v = s_kv[buf] + AK * KS;
-#pragma unroll
-        for (int j = 0; j < NL; j++) {
-            const int f = threadIdx.x + j * W * kWave;
-            const int row = f / (D / 4);
-            const int c4 = f - row * (D / 4);
-            *reinterpret_cast<float4*>(s_k + row * KS + 4 * c4) = pk[j];
-            *reinterpret_cast<float4*>(s_v + row * KS + 4 * c4) = pv[j];
-        }
-    };
-
-    // Tile t is computed from LDS buffer t % 2 while tile t + 1 waits in
-    // registers (loaded during tile t - 1) and tile t + 2 is loading.
-    if (k0 < k1) {
-        load_tile(k0);
-        store_tile(0);
-        if (k0 + AK < k1) load_tile(k0 + AK);
-        __syncthreads();
-    }
-    for (int t0 = k0; t0 < k1; t0 += AK) {
-        const float* const s_k = s_kv[cur];
-        const float* const s_v = s_kv[cur] + AK * KS;
-
-        // S^T for the KB key blocks: sv[4 kb + i] = score of key t0 + 16 kb + 4 g + i, query r.
-        float sv[4 * KB];
-#pragma unroll
-        for (int kb = 0; kb < KB; kb++) {
-            f32x4 c = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            const float* kr = s_k + (16 * kb + r) * KS + g * DQ;
-#pragma unroll
-            for (int s4 = 0; s4 < DQ; s4 += 4) {
-                const float4 kk = *reinterpret_cast<const float4*>(kr + s4);
-                c = __builtin_amdgcn_mfma_f32_16x16x4f32(kk.x, qv[s4], c, 0, 0, 0);
-                c = __builtin_amdgcn_mfma_f32_16x16x4f32(kk.y, qv[s4 + 1], c, 0, 0, 0);
-                c = __builtin_amdgcn_mfma_f32_16x16x4f32(kk.z, qv[s4 + 2], c, 0, 0, 0);
-                c = __builtin_amdgcn_mfma_f32_16x16x4f32(kk.w, qv[s4 + 3], c, 0, 0, 0);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int key = t0 + 16 * kb + 4 * g + i;
-                sv[4 * kb + i] = key < k1 ? c[i] : -INFINITY;
-            }
-        }
-        float mt = -INFINITY;
-#pragma unroll
-        for (int j = 0; j < 4 * KB; j++) mt = fmaxf(mt, sv[j]);
-        mt = fmaxf(mt, __shfl_xor(mt, 16));
-        mt = fmaxf(mt, __shfl_xor(mt, 32));
-        const float mn = fmaxf(m, mt);
-        const float ms = mn == -INFINITY ? 0.0f : mn;
-        const float alpha = fast_exp2(m - ms);
-        m = mn;
-        l *= alpha;
-#pragma unroll
-        for (int j = 0; j < 4 * KB; j++) {
-            sv[j] = fast_exp2(sv[j] - ms);
-            l += sv[j];
-        }
-        if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
-#pragma unroll
-            for (int c = 0; c < NB; c++) o[c] *= alpha;
-        }
-        // O^T += V^T P^T: step (kb, i) contracts keys 16 kb + 4 g + i (k index g).
-#pragma unroll
-        for (int kb = 0; kb < KB; kb++) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float* vr = s_v + (16 * kb + 4 * g + i) * KS + NB * r;
-                float vv[NB];
-                if constexpr (NB % 4 == 0) {
-#pragma unroll
-                    for (int c4 = 0; c4 < NB; c4 += 4) {
-                        const float4 x = *reinterpret_cast<const float4*>(vr + c4);
-                        vv[c4] = x.x;
-                        vv[c4 + 1] = x.y;
-                        vv[c4 + 2] = x.z;
-                        vv[c4 + 3] = x.w;
-                    }
-                } else {
-                    const float2 x = *reinterpret_cast<const float2*>(vr);
-                    vv[0] = x.x;
-                    vv[1] = x.y;
-                }
-#pragma unroll
-                for (int c = 0; c < NB; c++)
-                    o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[c], sv[4 * kb + i], o[c], 0, 0, 0);
-            }
-        }
-        // The next tile (in registers since the previous iteration) goes to the
-        // idle buffer, which every wave finished reading before the last
-        // barrier; the tile after it starts loading.  One barrier per tile.
-        if (t0 + AK < k1) {
-            store_tile(cur ^ 1);
-            if (t0 + 2 * AK < k1) load_tile(t0 + 2 * AK);
-        }
-        __syncthreads();
-        cur ^= 1;
-    }
-    l += __shfl_xor(l, 16);
-    l += __shfl_xor(l, 32);
-
-    // One split: the normalised output.  Several: the partial record of
-    // (split, query) -- unnormalised acc, and (m, l) -- for attention_merge.
-    const int q = q0 + r;
-    if (q < a.M) {
-        const bool whole = a.splits == 1;
-        const float inv = whole ? 1.0f / l : 1.0f;
-        float* const row = whole ? a.out + static_cast<size_t>(q) * D
-                                 : a.part_acc + (static_cast<size_t>(split) * a.M + q) * D;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            float* op = row + NB * (4 * g + i);
-            if constexpr (NB % 4 == 0) {
-#pragma unroll
-                for (int c4 = 0; c4 < NB; c4 += 4)
-                    *reinterpret_cast<float4*>(op + c4) = make_float4(o[c4][i] * inv, o[c4 + 1][i] * inv,
-                                                                      o[c4 + 2][i] * inv, o[c4 + 3][i] * inv);
-            } else {
-                *reinterpret_cast<float2*>(op) = make_float2(o[0][i] * inv, o[1][i] * inv);
-            }
-        }
-        if (!whole && g == 0)
-            *reinterpret_cast<float2*>(a.part_ml + (static_cast<size_t>(split) * a.M + q) * 2) = make_float2(m, l);
     }
 }
 
 // attention_direct<D, W, KW>: 9 to 64 queries (16 per wave, W query blocks)
-// on the same v_mfma_f32_16x16x4_f32 products as attention_mfma, but with no
-// LDS tile and no padded 64-query block: each wave streams keys from global
-// memory straight into its MFMA operands, 16 keys per block, the next block
+// on v_mfma_f32_16x16x4_f32 products (fp32 in and out), with no LDS tile and no
+// padded 64-query block: each wave streams keys from global memory straight into its MFMA operands, 16 keys per block, the next block
 // loading while the current one is computed.  KW waves share a query block's
 // split, taking every KW-th block of it, and meet in LDS at the end (part 0
 // rescales and adds the others' (m, l, o)), so the grid has KW times the waves
@@ -329,7 +124,7 @@ __global__ __launch_bounds__(W* kWave) void attention_mfma(const AttnArgs a) {
 // cover whole rows per lane group.  The W query blocks of a workgroup read
 // the same keys (L2 hits after the first).  Keys past the split's end read its last
 // row (in bounds); their scores are -inf and their V values zero.  Splits
-// write the (m, l, acc) records attention_merge combines, as attention_mfma.
+// write the (m, l, acc) records attention_merge combines.
 constexpr int kDirectBlock = 16;  // keys per block
 template <int D, int W, int KW>
 __global__ __launch_bounds__(W* KW* kWave) void attention_direct(const AttnArgs a) {
@@ -689,55 +484,23 @@ __global__ __launch_bounds__(W* kWave) void attention_rows(const AttnArgs a) {
     }
 }
 
-// Any d <= 1024: one wave per query row; scores of 64 keys per step, one per
-// lane (dot over d), online softmax over the steps, accumulator in LDS.
+// Any d <= 1024: one wave per query row (attention_row).
 constexpr int kGenWaves = 4;
 __global__ __launch_bounds__(kGenWaves* kWave) void attention_generic(const AttnArgs a) {
     extern __shared__ float sh[];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
     const int row = blockIdx.x * kGenWaves + wave;
-    const int d = a.d;
-    float* acc = sh + wave * d;
+    float* acc = sh + wave * a.d;
     if (row >= a.M) return;
-    for (int j = lane; j < d; j += kWave) acc[j] = 0.0f;
-    const float* q = a.q + static_cast<size_t>(row) * d;
-    float m = -INFINITY, l = 0.0f;
-    for (int t0 = 0; t0 < a.N; t0 += kWave) {
-        const int t = t0 + lane;
-        float s = -INFINITY;
-        if (t < a.N) {
-            const float* k = a.k + static_cast<size_t>(t) * d;
-            float dot = 0.0f;
-            for (int j = 0; j < d; j++) dot = fmaf(q[j], k[j], dot);
-            s = dot * a.scale_log2;
-        }
-        const float mn = fmaxf(m, wave_max(s));
-        const float alpha = fast_exp2(m - mn);
-        const float p = fast_exp2(s - mn);
-        l = l * alpha + wave_sum(p);
-        m = mn;
-        const int nt = min(kWave, a.N - t0);
-        // Dims in passes of 64 with every lane active, so the shuffles read
-        // live lanes; lanes past d carry zeros and store nothing.
-        for (int j0 = 0; j0 < d; j0 += kWave) {
-            const int j = j0 + lane;
-            const bool in = j < d;
-            float x = in ? acc[j] * alpha : 0.0f;
-            for (int u = 0; u < nt; u++) {
-                const float pu = __shfl(p, u);
-                x = fmaf(pu, in ? a.v[static_cast<size_t>(t0 + u) * d + j] : 0.0f, x);
-            }
-            if (in) acc[j] = x;
-        }
-    }
-    for (int j = lane; j < d; j += kWave) a.out[static_cast<size_t>(row) * d + j] = acc[j] / l;
+    float m, l;
+    attention_row(a, row, 0, a.N, acc, m, l);
+    for (int j = lane; j < a.d; j += kWave) a.out[static_cast<size_t>(row) * a.d + j] = acc[j] / l;
 }
 
 }  // namespace
 
-int attention_tuned_dim(int d) { return d == 32 || d == 64 || d == 128 || d == 256; }
-int attention_key_tile(int d) { return d >= 256 ? attention_tile<256>() : attention_tile<128>(); }
+int attention_rows_dim(int d) { return d == 32 || d == 64 || d == 128 || d == 256; }
 int attention_max_splits(int) { return kAttnMaxSplits; }
 int attention_direct_dim(int d) { return d == 64 || d == 128; }
 int attention_rows_queries(int M) {
@@ -765,15 +528,12 @@ int attention_rows_tile(int d, int qm) {
 }
 
 namespace {
-template <int D, int W>
-void launch_mfma_attention(const AttnArgs& a, int glog, hipStream_t stream) {
-    const dim3 grid(static_cast<unsigned>((a.M + 16 * W - 1) / (16 * W)), static_cast<unsigned>(a.splits));
-    hipLaunchKernelGGL((attention_mfma<D, W>), grid, dim3(W * kWave), 0, stream, a);
-    if (a.splits > 1) {
-        const dim3 mgrid(static_cast<unsigned>(
-            ((static_cast<long long>(a.M) * (D / 4) << glog) + kMergeThreads - 1) / kMergeThreads));
-        hipLaunchKernelGGL(attention_merge<D>, mgrid, dim3(kMergeThreads), 0, stream, a, glog);
-    }
+template <int D>
+void launch_merge(const AttnArgs& a, int glog, hipStream_t stream) {
+    if (a.splits <= 1) return;
+    const long long columns = static_cast<long long>(a.M) * (attention_record_dim(a.d) / 4);
+    const dim3 grid(static_cast<unsigned>(((columns << glog) + kMergeThreads - 1) / kMergeThreads));
+    hipLaunchKernelGGL(attention_merge<D>, grid, dim3(kMergeThreads), 0, stream, a, glog);
 }
 template <int D, int QM>
 void launch_rows_attention(const AttnArgs& a, int glog, hipStream_t stream) {
@@ -784,11 +544,7 @@ void launch_rows_attention(const AttnArgs& a, int glog, hipStream_t stream) {
         hipLaunchKernelGGL((attention_rows<D, QM, kRowsWavesShort>), grid, dim3(kRowsWavesShort * kWave), 0, stream, a);
     else
         hipLaunchKernelGGL((attention_rows<D, QM, kRowsWaves>), grid, dim3(kRowsWaves * kWave), 0, stream, a);
-    if (a.splits > 1) {
-        const dim3 mgrid(static_cast<unsigned>(
-            ((static_cast<long long>(a.M) * (D / 4) << glog) + kMergeThreads - 1) / kMergeThreads));
-        hipLaunchKernelGGL(attention_merge<D>, mgrid, dim3(kMergeThreads), 0, stream, a, glog);
-    }
+    launch_merge<D>(a, glog, stream);
 }
 template <int D>
 void launch_rows_attention_d(const AttnArgs& a, int glog, hipStream_t stream) {
@@ -803,47 +559,35 @@ template <int D, int W, int KW>
 void launch_direct_attention(const AttnArgs& a, int glog, hipStream_t stream) {
     const dim3 grid(static_cast<unsigned>((a.M + 16 * W - 1) / (16 * W)), static_cast<unsigned>(a.splits));
     hipLaunchKernelGGL((attention_direct<D, W, KW>), grid, dim3(W * KW * kWave), 0, stream, a);
-    if (a.splits > 1) {
-        const dim3 mgrid(static_cast<unsigned>(
-            ((static_cast<long long>(a.M) * (D / 4) << glog) + kMergeThreads - 1) / kMergeThreads));
-        hipLaunchKernelGGL(attention_merge<D>, mgrid, dim3(kMergeThreads), 0, stream, a, glog);
-    }
+    launch_merge<D>(a, glog, stream);
 }
 template <int D>
-void launch_mfma_attention_d(const AttnArgs& a, int glog, hipStream_t stream) {
-    if (a.qblock <= kRowsMaxQueries) {
-        launch_rows_attention_d<D>(a, glog, stream);
-        return;
-    }
-    if constexpr (D == 64 || D == 128) {
-        if (a.direct) {
-            // Up to 32 queries four waves share a query block's split; 33-64
-            // queries run as four query blocks of one wave each.
-            if (a.qblock == 16) launch_direct_attention<D, 1, 4>(a, glog, stream);
-            else if (a.qblock == 32) launch_direct_attention<D, 2, 4>(a, glog, stream);
-            else launch_direct_attention<D, 4, 1>(a, glog, stream);
-            return;
-        }
-    }
-    if constexpr (D <= 128) {  // at d = 256 a 4-wave block would need over 256 VGPRs
-        if (a.qblock == kAttnBlockNarrow) {
-            launch_mfma_attention<D, kAttnBlockNarrow / 16>(a, glog, stream);
-            return;
-        }
-    }
-    launch_mfma_attention<D, kAttnBlockWide / 16>(a, glog, stream);
+void launch_direct_attention_d(const AttnArgs& a, int glog, hipStream_t stream) {
+    // Up to 32 queries four waves share a query block's split; 33-64 queries
+    // run as four query blocks of one wave each.
+    if (a.qblock == 16) launch_direct_attention<D, 1, 4>(a, glog, stream);
+    else if (a.qblock == 32) launch_direct_attention<D, 2, 4>(a, glog, stream);
+    else launch_direct_attention<D, 4, 1>(a, glog, stream);
 }
 }  // namespace
 
 hipError_t launch_attention(const AttnArgs& a, hipStream_t stream) {
-    if (a.tuned && attention_tuned_dim(a.d)) {
+    if (a.tuned) {
         int glog = 0;  // lanes per merge group: at most 8 splits per lane, at most a wave
         while (glog < 6 && ((a.splits - 1) >> glog) >= 8) glog++;
-        switch (a.d) {
-            case 32: launch_mfma_attention_d<32>(a, glog, stream); break;
-            case 64: launch_mfma_attention_d<64>(a, glog, stream); break;
-            case 128: launch_mfma_attention_d<128>(a, glog, stream); break;
-            default: launch_mfma_attention_d<256>(a, glog, stream); break;
+        if (a.qblock <= kAttnRowsBlock) {
+            switch (a.d) {
+                case 32: launch_rows_attention_d<32>(a, glog, stream); break;
+                case 64: launch_rows_attention_d<64>(a, glog, stream); break;
+                case 128: launch_rows_attention_d<128>(a, glog, stream); break;
+                default: launch_rows_attention_d<256>(a, glog, stream); break;
+            }
+        } else if (a.direct) {
+            if (a.d == 64) launch_direct_attention_d<64>(a, glog, stream);
+            else launch_direct_attention_d<128>(a, glog, stream);
+        } else {
+            launch_attention_limbs(a, stream);
+            launch_merge<0>(a, glog, stream);
         }
         return hipGetLastError();
     }

@@ -643,11 +643,6 @@ DecodePlan paged_plan(const kvq_paged_decode_params* p) {
 
 // ---- dense attention ------------------------------------------------------
 
-// Workgroups the attention grid should reach before keys are split: one
-// round of resident matrix-core workgroups (8 waves each; at d = 128 the
-// register file holds one per CU, below that two).
-int attention_target_workgroups(int d) { return d >= 128 ? 256 : 512; }
-
 // The register-direct attention kernel (up to 64 queries, d = 64 or 128):
 // key splits per launch, KVQ_ATTN_DIRECT_SPLITS(M), but at least
 // min(blocks, 128) and at most half the 16-key blocks; up to 32 queries four
@@ -663,7 +658,7 @@ struct AttnPlan {
     bool tuned = false;
     bool direct = false;
     int splits = 1, chunk = 0;
-    int qblock = kvq::kAttnBlockWide;
+    int qblock = 0;
     size_t ml_bytes = 0, acc_bytes = 0;
     size_t bytes() const { return ml_bytes + acc_bytes; }
 };
@@ -675,16 +670,18 @@ bool attention_args_ok(int M, int N, int d, const void* q, const void* k, const 
     return N <= INT_MAX - 1024 && M <= INT_MAX - 1024;
 }
 
-AttnPlan attention_plan(int M, int N, int d, bool aligned, int requested) {
+// owned: the workspace is the library's.  A caller's own workspace was never
+// needed at head dims without a few-query kernel, so there it stays unsplit.
+AttnPlan attention_plan(int M, int N, int d, bool aligned, int requested, bool owned) {
     AttnPlan p;
-    p.tuned = kvq::attention_tuned_dim(d) && aligned;
+    p.tuned = d <= kvq::kAttnLimbMaxDim && aligned;
     p.chunk = N;
     if (!p.tuned) return p;  // the generic kernel runs unsplit
     // 9-16 queries over long key ranges at d = 32 or 256 also run the VALU
     // kernel, as 8-query blocks (M = 16, N = 65536, d = 256: 65.9 us against
     // 83.3 us in a padded matrix-core block); at d = 64 and 128 the
     // register-direct kernel below takes them.
-    int qm = kvq::attention_rows_queries(M);
+    int qm = kvq::attention_rows_dim(d) ? kvq::attention_rows_queries(M) : 0;
     // 5-8 queries at d = 64 and 128, and 3-4 at d = 64, go to the
     // register-direct kernel below (M = 8, N = 65536: 20.0 against 21.5 us at
     // d = 128, 11.2 against 16.2 at d = 64; M = 4, N = 65536, d = 64: 10.8
@@ -696,7 +693,7 @@ AttnPlan attention_plan(int M, int N, int d, bool aligned, int requested) {
     // at d = 128 from 16384 keys or with up to 32 queries, at d = 64 from
     // 32768 keys or with up to 8 queries.
     const bool direct_ok = M <= 64 && kvq::attention_direct_dim(d) && (d == 128 ? (N >= 16384 || M <= 32) : (N >= 32768 || M <= 8));
-    if (qm == 0 && M <= 2 * kvq::kAttnRowsBlock && N >= 65536 && !direct_ok) qm = kvq::kAttnRowsBlock;
+    if (qm == 0 && kvq::attention_rows_dim(d) && M <= 2 * kvq::kAttnRowsBlock && N >= 65536 && !direct_ok) qm = kvq::kAttnRowsBlock;
     if (qm > 0) {
         // A few queries: the VALU kernel, query blocks of qm, key splits to
         // fill KVQ_ATTN_ROWS_TARGET(qm) workgroups per query block.
@@ -732,31 +729,40 @@ AttnPlan attention_plan(int M, int N, int d, bool aligned, int requested) {
         }
         return p;
     }
-    const int tile = kvq::attention_key_tile(d);
+    // attention_limbs: query blocks of 64 (4 waves), 128 or 256 (8 waves, the
+    // second with two 16-query blocks per wave, d <= 128).  `work` counts
+    // 64-query x 32-key tiles.  A wide block splits K and V into limbs once for
+    // more queries, a narrow one starts faster and leaves fewer padded rows and
+    // fewer split records, so the line goes by how many tiles each of 256
+    // workgroups gets: 64 against 128 queries at d = 128 M = N = 1024 (2 tiles
+    // each) 14.8 / 17.7 us, M = N = 2048 (8) 27.5 / 26.7, M = 256 N = 16384 (8)
+    // 27.4 / 25.0, M = 1000 N = 3001 d = 96 (6) 19.6 / 22.3; 128 against 256 at
+    // M = 2048 N = 4096 d = 128 (16) 33.4 / 39.2, M = N = 4096 (32) d = 128
+    // 52.2 / 52.8, d = 64 37.0 / 34.4, M = N = 8192 d = 64 (128) 95.9 / 87.5.
+    const long long work = (static_cast<long long>(M) + 63) / 64 *
+                           ((static_cast<long long>(N) + kvq::kAttnLimbTile - 1) / kvq::kAttnLimbTile);
+    p.qblock = M <= 64 || work < 7 * 256                                      ? 64
+               : M > 512 && d <= 128 && work >= (d <= 64 ? 32 : 64) * 256LL ? 256
+                                                                              : 128;
+    // Key splits for one round of workgroups (one per CU; two at d <= 32: M = N
+    // = 8192 70.3 us with one, 61.7 with two), never a few more than a round
+    // (M = 700, N = 9000, d = 80 in 64-query blocks: 264 workgroups 41.9 us).
+    const int tile = (d <= 128 ? 2 : 1) * kvq::kAttnLimbTile;
     const long long tiles = (static_cast<long long>(N) + tile - 1) / tile;
-    const long long target = attention_target_workgroups(d);
-    // Splits for query blocks of qb: enough to fill the target, in whole key
-    // tiles, within the merge's limit.
-    auto splits_for = [&](int qb) {
-        const long long qblocks = (static_cast<long long>(M) + qb - 1) / qb;
-        const long long w = requested > 0 ? requested : (target + qblocks - 1) / qblocks;
-        return std::max(1LL, std::min({w, tiles, static_cast<long long>(kvq::attention_max_splits(d))}));
-    };
-    long long want = splits_for(kvq::kAttnBlockWide);
-    const long long wide_wgs = (static_cast<long long>(M) + kvq::kAttnBlockWide - 1) / kvq::kAttnBlockWide * want;
-    if (requested == 0 && wide_wgs < target && d <= 128) {
-        // The wide blocks leave CUs idle: narrow blocks double the grid.
-        p.qblock = kvq::kAttnBlockNarrow;
-        want = splits_for(kvq::kAttnBlockNarrow);
-    }
+    const long long target = d <= 32 ? 512 : 256;
+    const long long qblocks = (static_cast<long long>(M) + p.qblock - 1) / p.qblock;
+    long long want = requested > 0 ? requested : std::max(1LL, target / qblocks);
+    if (!owned && !kvq::attention_rows_dim(d)) want = 1;
+    want = std::max(1LL, std::min({want, tiles, static_cast<long long>(kvq::attention_max_splits(d))}));
     // The merge runs up to 64 lanes per 16-byte output column, indexed in int.
-    if (static_cast<long long>(M) * (d / 4) * 64 >= INT_MAX) want = 1;
+    if (static_cast<long long>(M) * (kvq::attention_record_dim(d) / 4) * 64 >= INT_MAX) want = 1;
     const long long chunk_tiles = (tiles + want - 1) / want;
     p.chunk = static_cast<int>(std::min<long long>(chunk_tiles * tile, N));
     p.splits = static_cast<int>((N + static_cast<long long>(p.chunk) - 1) / p.chunk);
     if (p.splits > 1) {
         p.ml_bytes = round_up(static_cast<size_t>(p.splits) * M * 2 * sizeof(float), kAlign);
-        p.acc_bytes = round_up(static_cast<size_t>(p.splits) * M * d * sizeof(float), kAlign);
+        p.acc_bytes =
+            round_up(static_cast<size_t>(p.splits) * M * kvq::attention_record_dim(d) * sizeof(float), kAlign);
     }
     return p;
 }
@@ -1054,7 +1060,7 @@ hipError_t kvq_prefill_quantize_launch(const kvq_prefill_params* p, hipStream_t 
 hipError_t attention_online_launch(const float* Q, const float* K, const float* V, float* output, int M, int N,
                                    int d, hipStream_t stream) {
     if (!attention_args_ok(M, N, d, Q, K, V, output)) return hipErrorInvalidValue;
-    const AttnPlan p = attention_plan(M, N, d, attention_aligned(Q, K, V, output), 0);
+    const AttnPlan p = attention_plan(M, N, d, attention_aligned(Q, K, V, output), 0, true);
     return checked_call(stream, [&] {
         return with_attention_workspace(p.bytes(), stream, [&](void* ws) {
             return attention_run(M, N, d, Q, K, V, output, 1.0f / sqrtf(static_cast<float>(d)), p, ws, stream);
@@ -1064,7 +1070,8 @@ hipError_t attention_online_launch(const float* Q, const float* K, const float* 
 
 size_t kvq_attention_workspace_size(const kvq_attention_params* p) {
     if (!p || !attention_args_ok(p->M, p->N, p->d, p->q, p->k, p->v, p->out) || p->num_splits < 0) return 0;
-    return attention_plan(p->M, p->N, p->d, attention_aligned(p->q, p->k, p->v, p->out), p->num_splits).bytes();
+    return attention_plan(p->M, p->N, p->d, attention_aligned(p->q, p->k, p->v, p->out), p->num_splits, false)
+        .bytes();
 }
 
 hipError_t kvq_attention_launch(const kvq_attention_params* p, void* workspace, size_t workspace_bytes,
@@ -1072,7 +1079,7 @@ hipError_t kvq_attention_launch(const kvq_attention_params* p, void* workspace, 
     if (!p || !attention_args_ok(p->M, p->N, p->d, p->q, p->k, p->v, p->out) || p->num_splits < 0)
         return hipErrorInvalidValue;
     const AttnPlan plan =
-        attention_plan(p->M, p->N, p->d, attention_aligned(p->q, p->k, p->v, p->out), p->num_splits);
+        attention_plan(p->M, p->N, p->d, attention_aligned(p->q, p->k, p->v, p->out), p->num_splits, false);
     if (plan.bytes() > 0 && (!workspace || workspace_bytes < plan.bytes() || !aligned16(workspace)))
         return hipErrorInvalidValue;
     const float scale = p->softmax_scale != 0.0f ? p->softmax_scale : 1.0f / sqrtf(static_cast<float>(p->d));
@@ -1107,7 +1114,7 @@ hipError_t kvq_paged_decode_plan(const kvq_paged_decode_params* p, kvq_plan_info
 hipError_t kvq_attention_plan(const kvq_attention_params* p, kvq_plan_info* info) {
     if (!info || !p || !attention_args_ok(p->M, p->N, p->d, p->q, p->k, p->v, p->out) || p->num_splits < 0)
         return hipErrorInvalidValue;
-    const AttnPlan plan = attention_plan(p->M, p->N, p->d, attention_aligned(p->q, p->k, p->v, p->out), p->num_splits);
+    const AttnPlan plan = attention_plan(p->M, p->N, p->d, attention_aligned(p->q, p->k, p->v, p->out), p->num_splits, false);
     kvq_plan_info r{};
     if (!plan.tuned) r.kernel = KVQ_KERNEL_ATTENTION_GENERIC;
     else if (plan.qblock <= kvq::kAttnRowsBlock) r.kernel = KVQ_KERNEL_ATTENTION_ROWS;

@@ -179,12 +179,9 @@ struct PrefillArgs {
 hipError_t launch_prefill(const PrefillArgs& a, int d, bool bf16, bool vec_ok, hipStream_t stream);
 hipError_t launch_fill_zero(void* p, size_t bytes, hipStream_t stream);
 
-// Dense fp32 attention (kvq_attention.hip): out = softmax(q k^T * scale) v.
-// Queries per matrix-core attention workgroup (16 per wave): 8 waves, or 4
-// when the wide blocks times the key splits cannot fill one round of
-// workgroups (few queries, or few keys to split).
-constexpr int kAttnBlockWide = 128;
-constexpr int kAttnBlockNarrow = 64;
+// Dense fp32 attention (kvq_attention.hip, kvq_attention_limbs.hpp): out = softmax(q k^T * scale) v.
+constexpr int kAttnLimbTile = 32;     // keys per LDS tile of attention_limbs
+constexpr int kAttnLimbMaxDim = 256;  // its largest head dim
 constexpr int kAttnRowsBlock = 8;     // queries per workgroup of the few-query kernel, at most
 
 struct AttnArgs {
@@ -193,20 +190,21 @@ struct AttnArgs {
     const float* v;    // [N, d]
     float* out;        // [M, d]
     float* part_ml;    // [splits, M, 2] partial (max in log2 units, sum)
-    float* part_acc;   // [splits, M, d] unnormalised partial accumulators
+    float* part_acc;   // [splits, M, attention_record_dim(d)] unnormalised partial accumulators
     int M, N, d;
     int splits, chunk;  // key splits (grid y) and keys per split (a multiple of the key tile)
-    int qblock;         // queries per workgroup: kAttnBlockWide or kAttnBlockNarrow (matrix cores),
-                        // or 1, 2, 4, 8 (few-query kernel, attention_rows)
+    int qblock;         // queries per workgroup: 64, 128 or 256 (attention_limbs), or 1, 2, 4, 8
+                        // (few-query kernel, attention_rows)
     bool direct;        // attention_direct: qblock 16, 32 or 64 queries (16 per wave), no LDS tiles;
                         // up to 32 queries four waves share each query block's split
     float scale_log2;   // softmax scale * log2(e)
-    bool tuned;         // a tuned kernel runs (tuned head dim and 16-byte aligned q, k, v, out);
+    bool tuned;         // a tuned kernel runs (d <= kAttnLimbMaxDim and 16-byte aligned q, k, v, out);
                         // otherwise attention_generic, unsplit
 };
-int attention_tuned_dim(int d);   // the matrix-core kernel handles head dim d
-int attention_key_tile(int d);    // keys per LDS tile of the matrix-core kernel at head dim d
-int attention_max_splits(int d);  // most key splits per matrix-core launch (tuned d)
+// Floats per partial accumulator: whole 16-byte columns for the merge.
+__host__ __device__ constexpr int attention_record_dim(int d) { return (d + 3) & ~3; }
+int attention_rows_dim(int d);    // attention_rows handles head dim d
+int attention_max_splits(int d);  // most key splits per launch
 int attention_direct_dim(int d);  // attention_direct handles head dim d
 int attention_rows_queries(int M);  // queries per workgroup of the few-query kernel (0: M too large)
 int attention_rows_tile(int d, int qm);  // keys per workgroup step of the few-query kernel (tuned d, qm queries)

@@ -323,7 +323,7 @@ const char* kvq_version(void);
 #define KVQ_KERNEL_DECODE_GENERIC 0   /* decode_generic: any head dim or alignment */
 #define KVQ_KERNEL_DECODE_VALU 1      /* decode_fast: per-lane FMAs */
 #define KVQ_KERNEL_DECODE_MFMA 2      /* decode_mfma: grouped-query heads on matrix cores */
-#define KVQ_KERNEL_ATTENTION_MFMA 3   /* attention_mfma: query blocks on matrix cores */
+#define KVQ_KERNEL_ATTENTION_MFMA 3   /* attention_limbs: query blocks on matrix cores, d <= 256 */
 #define KVQ_KERNEL_ATTENTION_ROWS 4   /* attention_rows: up to 8 queries per workgroup */
 #define KVQ_KERNEL_ATTENTION_GENERIC 5 /* attention_generic: any head dim or alignment */
 #define KVQ_KERNEL_ATTENTION_DIRECT 6  /* attention_direct: 9-64 queries, 16 per wave, no LDS tiles */

@@ -1,0 +1,95 @@
+"""attention_limbs (dense attention on bf16 matrix cores, three limbs per fp32
+value) at the edges of its tiles and dims, against float64.
+
+Bound: an output is a weighted mean of V rows, so it is at most max|V|; the
+limb products drop terms below 2^-24 of a product and the sums run in fp32, so
+scores of magnitude s (log2 units, s < 40 here) carry absolute errors of a few
+s * 2^-24, which are relative errors of the weights: 40 * 4 * 2^-24 < 1e-5, of
+max|V| < 6."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+import _gpu
+from _gpu import down, kvq, up
+
+pytestmark = pytest.mark.gpu
+BOUND = 6e-5
+
+
+def _problem(M, N, d, seed):
+    rng = np.random.default_rng(seed)
+    return [rng.standard_normal((n, d)).astype(np.float32) for n in (M, N, N)]
+
+
+def _exact(q, k, v):
+    s = q.astype(np.float64) @ k.astype(np.float64).T / math.sqrt(q.shape[1])
+    p = np.exp(s - s.max(1, keepdims=True))
+    return p @ v.astype(np.float64) / p.sum(1, keepdims=True)
+
+
+def _run(q, k, v, splits=None):
+    """attention_online's own splits, or kvq.attention with a request (which head dims other than 32, 64, 128 and 256
+    run unsplit)."""
+    gq, gk, gv = up(q), up(k), up(v)
+    out = _gpu.poisoned(q.shape)
+    info = kvq.attention_plan(kvq.attention_params(gq, gk, gv, out, num_splits=splits or 0))
+    assert info.kernel == kvq.KERNEL_ATTENTION_MFMA
+    if splits is None:
+        kvq.attention_online(gq, gk, gv, out)
+    else:
+        kvq.attention(gq, gk, gv, out, num_splits=splits)
+    torch.cuda.synchronize()
+    return down(out), info
+
+
+@pytest.mark.parametrize("d", [1, 17, 30, 33, 80, 96, 99, 112, 130, 160, 192, 255])
+@pytest.mark.parametrize("M,N,splits", [(1, 1, None), (17, 33, 0), (64, 31, None), (65, 257, None), (300, 95, 1),
+                                        (300, 950, None)])
+def test_head_dims(d, M, N, splits):
+    """Dims between the padded widths (32, 64, 96, 128, 192, 256), whole
+    16-byte columns and not; rows past M, keys past N, split and unsplit."""
+    q, k, v = _problem(M, N, d, 7 * d + M + N)
+    out, _ = _run(q, k, v, splits)
+    assert np.abs(out - _exact(q, k, v)).max() <= BOUND
+
+
+@pytest.mark.parametrize("M,N,d,qblock", [(65, 28640, 128, 64), (65, 28641, 128, 128), (1100, 14560, 64, 128),
+                                          (1089, 14561, 64, 256), (1089, 29121, 96, 256), (700, 9001, 256, 128)])
+def test_query_blocks(M, N, d, qblock):
+    """Each block size on both sides of the lines between them, with a ragged last split."""
+    q, k, v = _problem(M, N, d, M + N)
+    out, info = _run(q, k, v)
+    assert info.query_block == qblock
+    rows = np.random.default_rng(1).permutation(M)[:64]
+    assert np.abs(out[rows] - _exact(q[rows], k, v)).max() <= BOUND
+
+
+@pytest.mark.parametrize("M,N,d", [(70, 200, 96), (150, 9000, 64)])
+def test_rescaled_maximum(M, N, d):
+    """Scores that climb through the keys: the softmax reference moves again and again."""
+    q, k, v = _problem(M, N, d, 3)
+    k = (k * np.linspace(0.01, 3.0, N, dtype=np.float32)[:, None]).astype(np.float32)
+    out, _ = _run(q, k, v)
+    assert np.abs(out - _exact(q, k, v)).max() <= BOUND
+
+
+@pytest.mark.parametrize("splits", [1, None])
+def test_overflow_and_non_finite(splits):
+    """Values whose limbs overflow or are not finite take the fp32 rows: a key
+    whose score is -inf has weight 0, an infinite V element stays in its column."""
+    q, k, v = _problem(90, 300, 96, 11)
+    q = np.abs(q) + np.float32(1.0)
+    ref = _exact(q, np.delete(k, 40, 0), np.delete(v, 40, 0))
+    for big in (np.float32(-3.4e38), np.float32(-np.inf)):
+        kk = k.copy()
+        kk[40] = big
+        out, _ = _run(q, kk, v, splits)
+        assert np.abs(out - ref).max() <= BOUND
+    vv = v.copy()
+    vv[200, 5] = np.inf
+    out, _ = _run(q, k, vv, splits)
+    rest = np.arange(96) != 5
+    assert np.isposinf(out[:, 5]).all() and np.abs(out - _exact(q, k, v))[:, rest].max() <= BOUND
