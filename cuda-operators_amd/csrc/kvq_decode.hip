@@ -25,6 +25,7 @@
 //   Optionally wave 0 of the workgroup owning a sequence's last token
 //   quantises that token from fp32 (append) after its tiles, with no
 //   workgroup barrier, and attends to it from registers.
+//   PAD instances take the multiples of 16 from 48 to 240 between those dims.
 //
 // decode_generic: any head dim up to KVQ_MAX_HEAD_DIM and any alignment; one
 //   wave per (split, batch, query head), q and the accumulators in LDS.  It is
@@ -117,7 +118,15 @@ __device__ __forceinline__ void attend(const float (&qr)[SG][16], const int4 (&k
     }
 }
 
-template <int D, int SG, bool PAGED, bool FIT>
+// PAD: the head dim a.d is a multiple of 16 below D (and above D / 2).  Rows are
+// read at their own stride; the lanes past a.d hold zero q, read the row's last
+// 16 bytes again (no memory traffic) and store nothing.
+// Bound by HBM as the exact dims are, with 6 - 44 % of the lanes idle; these
+// shapes ran on decode_generic, which reads one byte per lane and waits on each
+// token in turn.  Before / after: B8 Hq32/Hkv32 d96 L 4096 with append 4417 /
+// 42.8 us (4.8 TB/s), H32 N 4099 d96 505 / 13.0 us, d192 737 / 17.4 us, B16
+// Hq32/Hkv8 d192 L 500-4000 6832 / 69 us, 16-token pages B8 H16 d80 1816 / 23 us.
+template <int D, int SG, bool PAGED, bool FIT, bool PAD>
 __global__ __launch_bounds__(kFastWaves* kWave) void decode_fast(const DecodeArgs a) {
     using Geo = FastGeom<D, SG>;
     constexpr int LPT = Geo::LPT;
@@ -133,6 +142,9 @@ __global__ __launch_bounds__(kFastWaves* kWave) void decode_fast(const DecodeArg
     const int wave = threadIdx.x / kWave;
     const int tg = lane / LPT;  // token slot within a wave load
     const int ds = lane % LPT;  // 16-element slice of the head dim
+    const int d = PAD ? a.d : D;
+    const bool own = !PAD || ds * 16 < d;                     // the lane's slice holds dims of the row
+    const int off16 = PAD ? min(ds * 16, d - 16) : ds * 16;  // its byte offset in a row
 
     SplitWork w;
     if constexpr (FIT) {
@@ -152,7 +164,7 @@ __global__ __launch_bounds__(kFastWaves* kWave) void decode_fast(const DecodeArg
     const int nsplit = w.nsplit;
 
     if (len == 0) {
-        for (int i = threadIdx.x; i < SG * D; i += blockDim.x) a.out[bhq0 * D + i] = 0.0f;
+        for (int i = threadIdx.x; i < SG * d; i += blockDim.x) a.out[bhq0 * d + i] = 0.0f;
         return;
     }
 
@@ -168,17 +180,19 @@ __global__ __launch_bounds__(kFastWaves* kWave) void decode_fast(const DecodeArg
     for (int j = 0; j < NE; j++) {
         const int e = lane + j * kWave;
         xnew[j] = 0.0f;
-        if (app && wave == 0 && e < 2 * D)
-            xnew[j] = (e < D ? a.k_new : a.v_new)[static_cast<size_t>(bh) * D + (e < D ? e : e - D)];
+        const int dim = e < D ? e : e - D;
+        if (app && wave == 0 && e < 2 * D && (!PAD || dim < d))
+            xnew[j] = (e < D ? a.k_new : a.v_new)[static_cast<size_t>(bh) * d + dim];
     }
 
     float qr[SG][16];
 #pragma unroll
     for (int h = 0; h < SG; h++) {
-        const float4* qp = reinterpret_cast<const float4*>(a.q + (bhq0 + h) * D + ds * 16);
+        const float4* qp = reinterpret_cast<const float4*>(a.q + (bhq0 + h) * d + off16);
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const float4 x = qp[j];
+            float4 x = qp[j];
+            if (!own) x = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             qr[h][4 * j + 0] = x.x;
             qr[h][4 * j + 1] = x.y;
             qr[h][4 * j + 2] = x.z;
@@ -194,7 +208,7 @@ __global__ __launch_bounds__(kFastWaves* kWave) void decode_fast(const DecodeArg
         for (int j = 0; j < 16; j++) acc[h][j] = 0.0f;
     }
 
-    // Cache rows (K/V row at byte row * D, scale at element row).  A wave
+    // Cache rows (K/V row at byte row * d, scale at element row).  A wave
     // tile's WSTEP tokens are consecutive rows in either layout: paged caches
     // run here only with power-of-two pages that are a multiple of WSTEP.
     const size_t row0 = static_cast<size_t>(bh) * a.cap;
@@ -209,16 +223,16 @@ __global__ __launch_bounds__(kFastWaves* kWave) void decode_fast(const DecodeArg
         float ks[U], vs[U];
     };
     auto load_tile = [&](Tile& T, int base, size_t r) {  // r: row of token `base`
-        const int8_t* kp = a.k + r * D + ds * 16;
-        const int8_t* vp = a.v + r * D + ds * 16;
+        const int8_t* kp = a.k + r * d + off16;
+        const int8_t* vp = a.v + r * d + off16;
         const float* ksp = a.ks + r;
         const float* vsp = a.vs + r;
         const int t_first = base + tg * U;
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const int tc = min(t_first + u, tend - 1) - base;
-            T.k[u] = load16_stream(kp + static_cast<ptrdiff_t>(tc) * D);
-            T.v[u] = load16_stream(vp + static_cast<ptrdiff_t>(tc) * D);
+            T.k[u] = load16_stream(kp + static_cast<ptrdiff_t>(tc) * d);
+            T.v[u] = load16_stream(vp + static_cast<ptrdiff_t>(tc) * d);
         }
         const float* ksu = ksp + (t_first - base);
         const float* vsu = vsp + (t_first - base);
@@ -346,8 +360,10 @@ __global__ __launch_bounds__(kFastWaves* kWave) void decode_fast(const DecodeArg
         const int tnew = len - 1;
         if (sgi == 0 && tg == 0) {
             const size_t rn = PAGED ? cache_row(a.pages, a.Hkv, a.cap, b, kvh, tnew) : row0 + tnew;
-            *reinterpret_cast<int4*>(a.k + rn * D + ds * 16) = kk1[0];
-            *reinterpret_cast<int4*>(a.v + rn * D + ds * 16) = vv1[0];
+            if (own) {
+                *reinterpret_cast<int4*>(a.k + rn * d + ds * 16) = kk1[0];
+                *reinterpret_cast<int4*>(a.v + rn * d + ds * 16) = vv1[0];
+            }
             if (ds == 0) {
                 a.ks[rn] = sk;
                 a.vs[rn] = sv;
@@ -397,6 +413,7 @@ __global__ __launch_bounds__(kFastWaves* kWave) void decode_fast(const DecodeArg
     for (int i = threadIdx.x; i < SG * D; i += blockDim.x) {
         const int h = i / D;
         const int dim = i - h * D;
+        if (PAD && dim >= d) continue;
         float M = -INFINITY;
 #pragma unroll
         for (int w = 0; w < kFastWaves; w++) M = fmaxf(M, s_ml[w][h][0]);
@@ -517,29 +534,29 @@ __global__ __launch_bounds__(kWave) void decode_generic(const DecodeArgs a) {
     }
 }
 
-template <int D, int SG>
+template <int D, int SG, bool PAD>
 void launch_fast_sg(const DecodeArgs& a, dim3 grid, dim3 block, hipStream_t stream) {
     // The in-kernel split plan (locate_fit) is built for SG <= 2 only: with
     // more heads per group the matrix-core kernel takes d = 128.
     if constexpr (SG <= 2) {
         if (a.fit_items > 0) {
-            if (a.pages.table) hipLaunchKernelGGL((decode_fast<D, SG, true, true>), grid, block, 0, stream, a);
-            else hipLaunchKernelGGL((decode_fast<D, SG, false, true>), grid, block, 0, stream, a);
+            if (a.pages.table) hipLaunchKernelGGL((decode_fast<D, SG, true, true, PAD>), grid, block, 0, stream, a);
+            else hipLaunchKernelGGL((decode_fast<D, SG, false, true, PAD>), grid, block, 0, stream, a);
             return;
         }
     }
-    if (a.pages.table) hipLaunchKernelGGL((decode_fast<D, SG, true, false>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((decode_fast<D, SG, false, false>), grid, block, 0, stream, a);
+    if (a.pages.table) hipLaunchKernelGGL((decode_fast<D, SG, true, false, PAD>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((decode_fast<D, SG, false, false, PAD>), grid, block, 0, stream, a);
 }
 
-template <int D>
+template <int D, bool PAD>
 hipError_t launch_fast_d(const DecodeArgs& a, const DecodePlan& p, hipStream_t stream) {
     const dim3 grid(static_cast<unsigned>(decode_grid(a, p)));
     const dim3 block(kFastWaves * kWave);
     switch (p.sg) {
-        case 1: launch_fast_sg<D, 1>(a, grid, block, stream); break;
-        case 2: launch_fast_sg<D, 2>(a, grid, block, stream); break;
-        case 4: launch_fast_sg<D, 4>(a, grid, block, stream); break;
+        case 1: launch_fast_sg<D, 1, PAD>(a, grid, block, stream); break;
+        case 2: launch_fast_sg<D, 2, PAD>(a, grid, block, stream); break;
+        case 4: launch_fast_sg<D, 4, PAD>(a, grid, block, stream); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -547,9 +564,15 @@ hipError_t launch_fast_d(const DecodeArgs& a, const DecodePlan& p, hipStream_t s
 
 }  // namespace
 
+int fast_padded_dim(int d) {
+    if (d == 32 || d == 64 || d == 128 || d == 256) return d;
+    if (d % 16 != 0 || d < 48 || d > 256) return 0;
+    return d < 64 ? 64 : d < 128 ? 128 : 256;
+}
+
 template <int SG>
 int tile_tokens_sg(int d) {
-    switch (d) {
+    switch (fast_padded_dim(d)) {
         case 32: return FastGeom<32, SG>::BSTEP;
         case 64: return FastGeom<64, SG>::BSTEP;
         case 128: return FastGeom<128, SG>::BSTEP;
@@ -600,11 +623,12 @@ hipError_t launch_decode(const DecodeArgs& a, const DecodePlan& p, hipStream_t s
         return hipSuccess;
     }
     if (p.kernel == Kernel::Valu) {
-        switch (a.d) {
-            case 32: err = launch_fast_d<32>(a, p, stream); break;
-            case 64: err = launch_fast_d<64>(a, p, stream); break;
-            case 128: err = launch_fast_d<128>(a, p, stream); break;
-            case 256: err = launch_fast_d<256>(a, p, stream); break;
+        const bool pad = fast_padded_dim(a.d) != a.d;
+        switch (fast_padded_dim(a.d)) {
+            case 32: err = launch_fast_d<32, false>(a, p, stream); break;
+            case 64: err = pad ? launch_fast_d<64, true>(a, p, stream) : launch_fast_d<64, false>(a, p, stream); break;
+            case 128: err = pad ? launch_fast_d<128, true>(a, p, stream) : launch_fast_d<128, false>(a, p, stream); break;
+            case 256: err = pad ? launch_fast_d<256, true>(a, p, stream) : launch_fast_d<256, false>(a, p, stream); break;
             default: return hipErrorInvalidValue;
         }
         if (err != hipSuccess) return err;

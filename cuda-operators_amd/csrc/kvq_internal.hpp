@@ -119,6 +119,7 @@ enum class Kernel {
 struct DecodePlan {
     Kernel kernel;
     bool fast;       // a tuned kernel (Valu or Mfma): 16-byte aligned rows
+    bool padded;     // Kernel::Valu at a head dim that its lanes pad
     int sg;          // query heads per workgroup (tuned kernels)
     int tile;        // tokens one workgroup iteration covers (tuned kernels; 0: generic)
     int nsg;         // G / sg, rounded up
@@ -213,6 +214,9 @@ hipError_t launch_attention(const AttnArgs& a, hipStream_t stream);
 // Tokens one workgroup iteration of the fast kernel covers for head dim d and
 // sg query heads per workgroup; 0 when the fast kernel does not support d.
 int fast_tile_tokens(int d, int sg);
+// The fast kernel's lane layout for head dim d: d itself, the next of 64, 128
+// and 256 (rows padded in registers), or 0 (not supported).
+int fast_padded_dim(int d);
 // Tokens one wave of the fast kernel covers per iteration (its tile).
 int fast_wave_tokens(int d, int sg);
 int fast_heads_per_group(int G);
