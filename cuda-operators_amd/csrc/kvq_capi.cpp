@@ -202,12 +202,17 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 // a paged cache only when no wave tile straddles a page;
 // ragged: per-sequence lengths on the device;
 // max_splits bounds the splits (scratch capacity of the reference ABI);
-// fused selects the arrival-counter merge (workspace holds counters).
+// fused selects the arrival-counter merge (workspace holds counters);
+// padding: tuned kernels may pad rows and head groups; without it they take
+// only the head dims and groups that fill their tiles.
 DecodePlan make_plan(int B, int Hq, int Hkv, int d, int max_len, bool aligned, bool quads, int page,
-                     bool ragged, int requested, int max_splits, bool fused) {
+                     bool ragged, int requested, int max_splits, bool fused, bool padding = true) {
     DecodePlan p{};
     const int G = Hq / Hkv;
-    const int sg_m = kvq::mfma_heads_per_group(G, d);
+    const int sg_m = padding                            ? kvq::mfma_heads_per_group(G, d)
+                     : (d != 64 && d != 128) || G % 4 != 0 ? 0
+                     : G % 8 == 0                          ? 8
+                                                           : 4;
     const int sg_v = kvq::fast_heads_per_group(G);
     const bool pow2 = page > 0 && (page & (page - 1)) == 0;
     const int wave_tokens = kvq::fast_wave_tokens(d, sg_v);
@@ -221,7 +226,8 @@ DecodePlan make_plan(int B, int Hq, int Hkv, int d, int max_len, bool aligned, b
         p.kernel = kvq::Kernel::Mfma;
         p.sg = sg_m;
         tile = kvq::mfma_tile_tokens();
-    } else if (aligned && valu_pages && kvq::fast_tile_tokens(d, sg_v) > 0) {
+    } else if (aligned && valu_pages && kvq::fast_tile_tokens(d, sg_v) > 0 &&
+               (padding || kvq::fast_padded_dim(d) == d)) {
         p.kernel = kvq::Kernel::Valu;
         p.sg = sg_v;
         p.padded = kvq::fast_padded_dim(d) != d;
@@ -598,10 +604,19 @@ bool decode_mfma_layout(const kvq_decode_params* p) {
     return aligned4(p->k_scale) && aligned4(p->v_scale) && p->capacity < (1 << 24);
 }
 
-DecodePlan decode_plan(const kvq_decode_params* p) {
-    return make_plan(p->batch, p->num_q_heads, p->num_kv_heads, p->head_dim, decode_max_len(p),
-                     decode_aligned(p), decode_mfma_layout(p), 0, p->lengths != nullptr, p->num_splits, INT_MAX,
-                     true);
+// The plan of a decode problem.  room: the size of a scratch array that cannot
+// grow (kvq_decode_launch_noalloc).  Padded tiles can need records where the
+// kernels that fill their tiles run without any (a ragged B700 Hq128/Hkv32 d48
+// step: 18 MB against none); a step too large for the array with them takes
+// the unpadded plan.
+DecodePlan decode_plan(const kvq_decode_params* p, size_t room = SIZE_MAX) {
+    auto plan = [&](bool quads, bool padding) {
+        return make_plan(p->batch, p->num_q_heads, p->num_kv_heads, p->head_dim, decode_max_len(p), decode_aligned(p),
+                         quads, 0, p->lengths != nullptr, p->num_splits, INT_MAX, true, padding);
+    };
+    const DecodePlan padded = plan(decode_mfma_layout(p), true);
+    if (plan_bytes(padded) <= room) return padded;
+    return plan(decode_mfma_layout(p) && aligned16(p->k_scale) && aligned16(p->v_scale) && p->capacity % 4 == 0, false);
 }
 
 bool paged_params_ok(const kvq_paged_decode_params* p) {
@@ -903,7 +918,7 @@ hipError_t kvq_decode_launch(const kvq_decode_params* p, void* workspace, size_t
 
 hipError_t kvq_decode_launch_noalloc(const kvq_decode_params* p, hipStream_t stream) {
     if (!decode_params_ok(p)) return hipErrorInvalidValue;
-    const DecodePlan plan = decode_plan(p);
+    const DecodePlan plan = decode_plan(p, KVQ_NOALLOC_SCRATCH_BYTES);
     const size_t need = plan_bytes(plan);
     if (need > KVQ_NOALLOC_SCRATCH_BYTES) return hipErrorInvalidValue;  // beyond the fixed scratch array
     return checked_call(stream, [&] {
