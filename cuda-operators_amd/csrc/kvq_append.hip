@@ -86,13 +86,19 @@ __device__ __forceinline__ float lanes_max(float x) {
 // rows, so the resident workgroups read and write one moving window of the
 // input and the cache (a grid-stride loop over 8192 workgroups, every
 // workgroup a quarter of the rows apart, was 10% slower for fp32).
+// PAD: a row of d < D elements, whole 16-byte pieces; the lanes past its last
+// piece reread that piece (the same cache line, and the row maximum is the
+// same) and store nothing.  Bound by the mixed read / write stream like the
+// full rows; against one wave per row with 2- or 4-byte loads, B16 Hkv8 L2047:
+// d = 96 bf16 159.7 -> 34.7 us (0.96 -> 4.41 TB/s), fp32 158.7 -> 49.7 us
+// (5.11 TB/s), d = 112 fp32 242.7 -> 63.5 us; one 33-token prompt 10.6 -> 10.2 us.
 constexpr int kPrefillWaves = 4;
 constexpr unsigned kPrefillMaxGroups = 1u << 20;
 template <bool BF16>
 constexpr int prefill_unroll() { return BF16 ? 4 : 8; }
 
-template <int D, bool BF16>
-__global__ __launch_bounds__(kPrefillWaves* kWave) void prefill_kernel(const PrefillArgs a) {
+template <int D, bool BF16, bool PAD>
+__global__ __launch_bounds__(kPrefillWaves* kWave) void prefill_kernel(const PrefillArgs a, int pad_d) {
     constexpr int EPL = BF16 ? 8 : 4;
     constexpr int LPR = D / EPL;
     constexpr int RPW = kWave / LPR;
@@ -101,7 +107,9 @@ __global__ __launch_bounds__(kPrefillWaves* kWave) void prefill_kernel(const Pre
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
     const int slot = lane / LPR;  // row within a wave load
-    const int ls = lane % LPR;    // 16-byte piece of the row
+    const int d = PAD ? pad_d : D;
+    const int ls = PAD ? min(lane % LPR, d / EPL - 1) : lane % LPR;  // 16-byte piece of the row
+    const bool owner = !PAD || ls == lane % LPR;
     const int kv = blockIdx.y;    // 0: K rows, 1: V rows
     const char* x = static_cast<const char*>(kv ? a.v_new : a.k_new);
     int8_t* qo = kv ? a.v : a.k;
@@ -123,7 +131,7 @@ __global__ __launch_bounds__(kPrefillWaves* kWave) void prefill_kernel(const Pre
         for (int u = 0; u < kPrefillU; u++) {
             row[u] = r0 + u * RPW + slot;
             const unsigned rc = min(row[u], a.rows - 1);
-            raw[u] = *reinterpret_cast<const int4*>(x + (static_cast<size_t>(rc) * D + ls * EPL) * ESZ);
+            raw[u] = *reinterpret_cast<const int4*>(x + (static_cast<size_t>(rc) * d + ls * EPL) * ESZ);
         }
         // Each row's destination: (b, kv head, token) from the row index,
         // then the cache row.  start[b] and the page-table entries come
@@ -174,22 +182,23 @@ __global__ __launch_bounds__(kPrefillWaves* kWave) void prefill_kernel(const Pre
 #pragma unroll
             for (int i = 0; i < EPL; i++) am = fmaxf(am, fabsf(e[i]));
             const float scale = quant_scale(lanes_max<LPR>(am));
-            if (orow[u] < 0) continue;
+            if (orow[u] < 0 || !owner) continue;
             const size_t o = static_cast<size_t>(orow[u]);
             int qv[EPL];
             quant_row<EPL>(e, scale, qv);
             if constexpr (BF16) {
                 const int2 pk = make_int2(pack4(qv[0], qv[1], qv[2], qv[3]), pack4(qv[4], qv[5], qv[6], qv[7]));
-                *reinterpret_cast<int2*>(qo + o * D + ls * EPL) = pk;
+                *reinterpret_cast<int2*>(qo + o * d + ls * EPL) = pk;
             } else {
-                *reinterpret_cast<int*>(qo + o * D + ls * EPL) = pack4(qv[0], qv[1], qv[2], qv[3]);
+                *reinterpret_cast<int*>(qo + o * d + ls * EPL) = pack4(qv[0], qv[1], qv[2], qv[3]);
             }
             if (ls == 0) so[o] = scale;
         }
     }
 }
 
-// Any head dim / alignment: one wave per row, lanes striding over it.
+// Any head dim / alignment: one wave per row, lanes striding over it, one
+// element per load.
 template <bool BF16>
 __global__ __launch_bounds__(kPrefillWaves* kWave) void prefill_generic_kernel(const PrefillArgs a, int d) {
     const int lane = threadIdx.x & (kWave - 1);
@@ -255,21 +264,21 @@ hipError_t launch_prefill_t(const PrefillArgs& a, int d, bool vec_ok, hipStream_
     };
     const dim3 block(kPrefillWaves * kWave);
     constexpr int EPL = BF16 ? 8 : 4;
-    if (vec_ok) {
-        switch (d) {
-#define KVQ_PREFILL_CASE(DD)                                                                        \
-    case DD:                                                                                        \
-        hipLaunchKernelGGL((prefill_kernel<DD, BF16>),                                              \
-                           grid_for(kPrefillWaves * (kWave / (DD / EPL)) * prefill_unroll<BF16>()), block, 0, \
-                           stream, a);                                                              \
-        return hipGetLastError();
-            KVQ_PREFILL_CASE(32)
-            KVQ_PREFILL_CASE(64)
-            KVQ_PREFILL_CASE(128)
-            KVQ_PREFILL_CASE(256)
+    // Rows of whole 16-byte pieces up to 256 elements; other lengths and
+    // misaligned rows go to the generic kernel.
+    if (vec_ok && d <= 256 && d % EPL == 0) {
+#define KVQ_PREFILL_CASE(DD)                                                                               \
+    if (d <= DD) {                                                                                         \
+        const dim3 grid = grid_for(kPrefillWaves * (kWave / (DD / EPL)) * prefill_unroll<BF16>());         \
+        if (d == DD) hipLaunchKernelGGL((prefill_kernel<DD, BF16, false>), grid, block, 0, stream, a, d);  \
+        else hipLaunchKernelGGL((prefill_kernel<DD, BF16, true>), grid, block, 0, stream, a, d);           \
+        return hipGetLastError();                                                                          \
+    }
+        KVQ_PREFILL_CASE(32)
+        KVQ_PREFILL_CASE(64)
+        KVQ_PREFILL_CASE(128)
+        KVQ_PREFILL_CASE(256)
 #undef KVQ_PREFILL_CASE
-            default: break;
-        }
     }
     hipLaunchKernelGGL((prefill_generic_kernel<BF16>), grid_for(kPrefillWaves), block, 0, stream, a, d);
     return hipGetLastError();
