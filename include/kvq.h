@@ -36,8 +36,8 @@
 extern "C" {
 #endif
 
-/* Largest head_dim any entry point accepts (head_dim in {32,64,128,256} runs
- * the tuned kernels; any other value up to this bound runs a generic kernel). */
+/* Largest head_dim any entry point accepts (32 and multiples of 16 from 48 to
+ * 256 run the tuned kernels; any other value up to this bound runs a generic kernel). */
 #define KVQ_MAX_HEAD_DIM 4096
 
 /* Longest sequence any decode entry point attends to, in tokens: seq_len of
