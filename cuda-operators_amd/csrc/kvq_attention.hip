@@ -140,7 +140,7 @@ __global__ __launch_bounds__(W* KW* kWave) void attention_direct(const AttnArgs 
     const int split = blockIdx.y;
     const int q0 = blockIdx.x * (16 * W) + wq * 16;
     const int k0 = split * a.chunk;
-    const int k1 = min(a.N, k0 + a.chunk);
+    const int k1 = attention_split_end(a.N, split, a.chunk);
 
     float qv[DQ];
     {
@@ -351,7 +351,7 @@ __global__ __launch_bounds__(W* kWave) void attention_rows(const AttnArgs a) {
     const int q0 = blockIdx.x * QM;
     const int split = blockIdx.y;
     const int k0 = split * a.chunk;
-    const int k1 = min(a.N, k0 + a.chunk);
+    const int k1 = attention_split_end(a.N, split, a.chunk);
 
     // Element 4j + i of a lane's dims is dim 4(jL + ds) + i.
     float qv[QM][E], acc[QM][E], m[QM], l[QM];

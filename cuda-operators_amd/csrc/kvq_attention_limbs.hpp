@@ -94,7 +94,7 @@ __global__ __launch_bounds__(W* kWave) void attention_limbs(const AttnArgs a) {
     const int split = blockIdx.y;
     const int q0 = blockIdx.x * (16 * QB * W) + wave * (16 * QB);
     const int k0 = split * a.chunk;
-    const int k1 = min(a.N, k0 + a.chunk);
+    const int k1 = attention_split_end(a.N, split, a.chunk);
     const int tiles = (k1 - k0 + AK - 1) / AK;
 
     // The first half of the waves loads and stores K tiles, the second V tiles,

@@ -202,6 +202,12 @@ struct AttnArgs {
     bool tuned;         // a tuned kernel runs (d <= kAttnLimbMaxDim and 16-byte aligned q, k, v, out);
                         // otherwise attention_generic, unsplit
 };
+// End of split `split`'s keys, [split * chunk, end).  The last split's chunk may
+// reach past INT_MAX (one query at d = 1 over INT_MAX - 1024 keys: 256 splits of
+// 2^23), so the comparison is made on what is left of N.
+__host__ __device__ constexpr int attention_split_end(int N, int split, int chunk) {
+    return N - split * chunk < chunk ? N : split * chunk + chunk;
+}
 // Floats per partial accumulator: whole 16-byte columns for the merge.
 __host__ __device__ constexpr int attention_record_dim(int d) { return (d + 3) & ~3; }
 int attention_rows_dim(int d);    // attention_rows handles head dim d

@@ -378,6 +378,27 @@ void attention_plans() {
     }
 }
 
+// Key splits of whole tiles, as the attention planner cuts them, cover [0, N)
+// in order, in 32-bit arithmetic, up to the largest N that is accepted.
+void attention_split_bounds() {
+    for (int N : {1, 63, 4097, 1 << 24, (1 << 30) + 1, INT_MAX - 1024 - (1 << 23), INT_MAX - 1025, INT_MAX - 1024}) {
+        for (long tile : {16L, 32L, 64L, 128L, 512L}) {
+            for (long want : {1L, 2L, 7L, 255L, 256L, 512L, 1024L}) {
+                const long tiles = (N + tile - 1) / tile;
+                const int chunk = static_cast<int>(std::min<long>((tiles + want - 1) / want * tile, N));
+                const int splits = static_cast<int>((static_cast<long>(N) + chunk - 1) / chunk);
+                int at = 0;
+                for (int i = 0; i < splits; i++) {
+                    const int end = kvq::attention_split_end(N, i, chunk);
+                    expect(i * chunk == at && end > at && end <= N, "split bounds", N, chunk, i, end);
+                    at = end;
+                }
+                expect(at == N, "the splits end at N", N, chunk, splits, at);
+            }
+        }
+    }
+}
+
 void writers() {
     // Append / paged append / prefill / quantize: single bad fields.
     for (int which = 0; which < 6; which++) {
@@ -469,6 +490,7 @@ int main() {
     paged_plans();
     paged_bounds();
     attention_plans();
+    attention_split_bounds();
     writers();
     if (g_fails) {
         std::printf("FAILED %ld of %ld checks\n", g_fails, g_checks);
