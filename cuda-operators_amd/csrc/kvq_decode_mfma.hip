@@ -78,6 +78,9 @@ __device__ __forceinline__ f16x8 i8x8_to_f16(i32x2 v) {
     return f16x8{h0.x, h0.y, h1.x, h1.y, h2.x, h2.y, h3.x, h3.y};
 }
 
+// The larger of two floats, NaN if either is (v_maximum3_f32).
+__device__ __forceinline__ float max_or_nan(float x, float y) { return __builtin_elementwise_maximum(x, y); }
+
 // The power of two above x >= 0 (0 for 0): dividing by it and multiplying back is exact.
 __device__ __forceinline__ float pow2_above(float x) {
     return x > 0.0f ? __uint_as_float((__float_as_uint(x) & 0x7f800000u) + 0x00800000u) : 0.0f;
@@ -248,13 +251,16 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
     auto prepare_q = [&]() {
         float qmax = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 16 * NJ; i++) qmax = fmaxf(qmax, fabsf(qv[i]));
-        qmax = fmaxf(qmax, __shfl_xor(qmax, 16));
-        qmax = fmaxf(qmax, __shfl_xor(qmax, 32));
+        for (int i = 0; i < 16 * NJ; i++) qmax = max_or_nan(qmax, fabsf(qv[i]));
+        qmax = max_or_nan(qmax, __shfl_xor(qmax, 16));
+        qmax = max_or_nan(qmax, __shfl_xor(qmax, 32));
         int qexp = 0;
         frexpf(qmax, &qexp);  // qmax < 2^qexp
         const int E = qmax > 0.0f ? min(max(kQBits - qexp, -100), 126) : 0;
-        qs = ldexpf(1.0f, -E) * a.scale_log2;
+        // A row with an element that is not finite has no fixed-point value;
+        // its scores are NaN, infinite or all -inf, so its output is NaN
+        // whatever the limbs hold: qs = NaN.
+        qs = fmaf(qmax, 0.0f, ldexpf(1.0f, -E)) * a.scale_log2;
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
             int limb[kLimbs][16];
@@ -936,13 +942,16 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
     auto prepare_q = [&]() {
         float qmax = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 16 * NJ; i++) qmax = fmaxf(qmax, fabsf(qv[i]));
-        qmax = fmaxf(qmax, __shfl_xor(qmax, 16));
-        qmax = fmaxf(qmax, __shfl_xor(qmax, 32));
+        for (int i = 0; i < 16 * NJ; i++) qmax = max_or_nan(qmax, fabsf(qv[i]));
+        qmax = max_or_nan(qmax, __shfl_xor(qmax, 16));
+        qmax = max_or_nan(qmax, __shfl_xor(qmax, 32));
         int qexp = 0;
-        frexpf(qmax, &qexp);
+        frexpf(qmax, &qexp);  // qmax < 2^qexp
         const int E = qmax > 0.0f ? min(max(kQBits - qexp, -100), 126) : 0;
-        qs = ldexpf(1.0f, -E) * a.scale_log2;
+        // A row with an element that is not finite has no fixed-point value;
+        // its scores are NaN, infinite or all -inf, so its output is NaN
+        // whatever the limbs hold: qs = NaN.
+        qs = fmaf(qmax, 0.0f, ldexpf(1.0f, -E)) * a.scale_log2;
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
             int limb[kLimbs][16];
