@@ -23,8 +23,8 @@
 // * softmax: the running max m of s = (dot * k_scale) * softmax_scale * log2 e
 //   gives p = exp2(s - m) and the denominator; the PV weights are
 //   w = p * v_scale * 2^15 / vref, with vref the running max of |v_scale|, so
-//   |w| <= 2^15 whatever the scale magnitudes (PAD: vref is the power of two
-//   above that max, so scaling by it rounds nothing).  A tile that raises m or vref
+//   |w| <= 2^15 whatever the scale magnitudes (PAD: powers of two, next_vref).
+//   A tile that raises m or vref
 //   rescales the accumulator once (skipped when no row of the wave changed).
 // * PV on v_mfma_f32_16x16x32_f16 computing O^T[dim, row] += V^T P: the
 //   weights are split into f16 hi + lo rows (rows n < G.. hold hi, the next G
@@ -58,7 +58,6 @@ typedef __attribute__((address_space(3))) i32x2 lds_i32x2;
 
 constexpr int kMWaves = kMfmaWaves;  // waves per workgroup
 constexpr int kMTile = kMfmaTile;  // tokens per wave tile
-constexpr float kPScale = 32768.0f;  // PV weights are formed in (-2^15, 2^15) before the f16 split
 constexpr int kMBStep = kMTile * kMWaves;
 
 // 8 signed bytes -> 8 f16 (exact): bias each byte to unsigned, place it under
@@ -81,9 +80,38 @@ __device__ __forceinline__ f16x8 i8x8_to_f16(i32x2 v) {
 // The larger of two floats, NaN if either is (v_maximum3_f32).
 __device__ __forceinline__ float max_or_nan(float x, float y) { return __builtin_elementwise_maximum(x, y); }
 
-// The power of two above x >= 0 (0 for 0): dividing by it and multiplying back is exact.
-__device__ __forceinline__ float pow2_above(float x) {
-    return x > 0.0f ? __uint_as_float((__float_as_uint(x) & 0x7f800000u) + 0x00800000u) : 0.0f;
+// PV weights are w = p * v_scale * weight_scale / vref, |w| <= 2^15.  vref after
+// a tile whose largest |v_scale|, or kVrefMin if that is larger, is vmax; also
+// winv = weight_scale / vref and ratio = old vref / new.  With the floor winv stays finite for V rows of any size (with the reciprocal of a smaller
+// one infinite weights left NaN in the accumulator from 2^-113 down).
+// PAD: vref is the power of two at or below the largest |v_scale|, 2^127 at
+// most whatever the scales hold, so scaling by it rounds nothing and winv is a
+// subtraction of exponents.
+constexpr float kVrefMin = 0x1p-110f;
+template <bool PAD>
+constexpr float weight_scale() { return PAD ? 0x1p14f : 0x1p15f; }
+template <bool PAD>
+__device__ __forceinline__ float next_vref(float vref, float vmax, float& winv, float& ratio) {
+    if constexpr (PAD) {
+        const unsigned e = min(max(__float_as_uint(vmax) & 0x7f800000u, __float_as_uint(vref)), 0x7f000000u);
+        winv = __uint_as_float((268u << 23) - e);  // 2^14 / 2^n has the exponent field 14 - n + 127
+        ratio = vref * winv * (1.0f / weight_scale<PAD>());
+        return __uint_as_float(e);
+    } else {
+        const float vn = fmaxf(vref, vmax);
+        const float rvn = __builtin_amdgcn_rcpf(vn);  // v_rcp_f32, 1 ulp
+        winv = weight_scale<PAD>() * rvn;
+        ratio = vref * rvn;
+        return vn;
+    }
+}
+
+// The low half of a PV weight.  PAD: finite where the weight is infinite (an
+// infinite scale), so that the sum of both halves' products is infinite, not NaN.
+template <bool PAD>
+__device__ __forceinline__ _Float16 low_part(float w, _Float16 hi) {
+    const float lo = w - static_cast<float>(hi);
+    return static_cast<_Float16>(PAD ? __builtin_amdgcn_fmed3f(lo, -16.0f, 16.0f) : lo);
 }
 
 __device__ __forceinline__ int pack_bytes(const int* b) {
@@ -285,7 +313,7 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
     // row): the score max m (log2 units), the denominator lsum, and vref, the
     // running max of |v_scale| that keeps the PV weights p * v_scale / vref in
     // [-1, 1].  acc[c] holds O^T[16c + 4g + i][row r] in units of
-    // vref / kPScale.
+    // vref / weight_scale.
     float m = -INFINITY, lsum = 0.0f, vref = 0.0f;
     f32x4 acc[NB];
 #pragma unroll
@@ -485,7 +513,7 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
         // Scores in log2 units, k-slot order s*4 + i: the low limbs combine
         // exactly in int32 ((C1 << 8) + C2 < 2^30), the top limb in fp32.
         float sc[8], vsv[8];
-        float mt = -INFINITY, vmax = 0.0f;
+        float mt = -INFINITY, vmax = kVrefMin;
 #pragma unroll
         for (int s = 0; s < 2; s++) {
 #pragma unroll
@@ -523,18 +551,16 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
         const float mn = fmaxf(m, mt);
         const float ms = mn == -INFINITY ? 0.0f : mn;
         const float alpha = fast_exp2(m - ms);
-        const float vn = fmaxf(vref, PAD ? pow2_above(vmax) : vmax);
-        const float rvn = vn > 0.0f ? __builtin_amdgcn_rcpf(vn) : 0.0f;  // v_rcp_f32, 1 ulp (PAD: exact)
-        const float f = vn > 0.0f ? alpha * (vref * rvn) : alpha;
-        const float winv = kPScale * rvn;
+        float winv, ratio;
+        vref = next_vref<PAD>(vref, vmax, winv, ratio);
+        const float f = alpha * ratio;
         m = mn;
-        vref = vn;
         if (__builtin_amdgcn_ballot_w64(f != 1.0f) != 0) {  // a row's max or vref moved
 #pragma unroll
             for (int c = 0; c < NB; c++) acc[c] *= f;
         }
         // P^T as the PV B operand: row r takes the hi or lo f16 part of
-        // w = p * v_scale * kPScale / vref.
+        // w = p * v_scale * weight_scale / vref.
         float ps = 0.0f;
         f16x8 pb;
 #pragma unroll
@@ -543,7 +569,7 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
             ps += p;
             const float w = p * (vsv[k] * winv);
             const _Float16 hi = static_cast<_Float16>(w);
-            const _Float16 lo = static_cast<_Float16>(w - static_cast<float>(hi));
+            const _Float16 lo = low_part<PAD>(w, hi);
             pb[k] = lo_row ? lo : hi;
         }
         lsum = lsum * alpha + ps;
@@ -594,7 +620,7 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
     lsum += __shfl_xor(lsum, 16);
     lsum += __shfl_xor(lsum, 32);
     __syncthreads();  // every wave is done with its V tiles (s_acc reuses them)
-    const float fct = vref * (1.0f / kPScale);
+    const float fct = vref * (1.0f / weight_scale<PAD>());
 #pragma unroll
     for (int c = 0; c < NB; c++) {
 #pragma unroll
@@ -1185,7 +1211,7 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
             }
         }
         float sc[8], vsv[8];
-        float mt = -INFINITY, vmax = 0.0f;
+        float mt = -INFINITY, vmax = kVrefMin;
 #pragma unroll
         for (int s = 0; s < 2; s++) {
 #pragma unroll
@@ -1220,12 +1246,10 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
         const float mn = fmaxf(m, mt);
         const float ms = mn == -INFINITY ? 0.0f : mn;
         const float alpha = fast_exp2(m - ms);
-        const float vn = fmaxf(vref, PAD ? pow2_above(vmax) : vmax);
-        const float rvn = vn > 0.0f ? __builtin_amdgcn_rcpf(vn) : 0.0f;  // v_rcp_f32, 1 ulp (PAD: exact)
-        const float f = vn > 0.0f ? alpha * (vref * rvn) : alpha;
-        const float winv = kPScale * rvn;
+        float winv, ratio;
+        vref = next_vref<PAD>(vref, vmax, winv, ratio);
+        const float f = alpha * ratio;
         m = mn;
-        vref = vn;
         if (__builtin_amdgcn_ballot_w64(f != 1.0f) != 0) {
 #pragma unroll
             for (int c = 0; c < NB; c++) acc[c] *= f;
@@ -1238,7 +1262,7 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
             ps += p;
             const float w = p * (vsv[k] * winv);
             const _Float16 hi = static_cast<_Float16>(w);
-            const _Float16 lo = static_cast<_Float16>(w - static_cast<float>(hi));
+            const _Float16 lo = low_part<PAD>(w, hi);
             pb[k] = lo_row ? lo : hi;
         }
         lsum = lsum * alpha + ps;
@@ -1256,11 +1280,13 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
         float lt = lsum;
         lt += __shfl_xor(lt, 16);
         lt += __shfl_xor(lt, 32);
-        const float fct = vref * (1.0f / kPScale);
+        const float fct = vref * (1.0f / weight_scale<PAD>());
         const bool writer = r < hc;
         const size_t row = static_cast<size_t>(b) * a.Hq + hq0 + r;
         const size_t rec = (static_cast<size_t>(gw) + b) * a.Hq + hq0 + r;
-        const float sc = complete ? fct / lt : fct;
+        // (PAD scales by the power of two apart: fct / lt is subnormal for tiny V rows.)
+        const float sc = PAD ? (complete ? 1.0f / lt : 1.0f) : complete ? fct / lt : fct;
+        const float unit = PAD ? fct : 1.0f;
         const buf_rsrc recr = make_rsrc(a.part_acc + (static_cast<size_t>(gw) + b) * a.Hq * d, a.Hq * d * 4u);
 #pragma unroll
         for (int c = 0; c < NB; c++) {
@@ -1269,7 +1295,7 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
             for (int i = 0; i < 4; i++)
                 o[i] = (acc[c][i] + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc[c][i]),
-                                                                                 0x100 + G, 0xF, 0xF, false))) * sc;
+                                                                                 0x100 + G, 0xF, 0xF, false))) * unit * sc;
             if (writer && (!PAD || 16 * c < d)) {
                 if (complete) {
 #pragma unroll

@@ -71,3 +71,73 @@ def test_non_finite_queries(o, name, bad):
     got = _decode(rng, p, lengths, page)
     assert np.isnan(got[rows]).all()
     assert_close(got[~rows], want[~rows], what=name)
+
+
+def _relative_error(got, p, lengths):
+    """Largest error of an output row over the row's norm, against float64."""
+    want = textbook_decode_f64(p["q"], p["k"], p["v"], p["ks"], p["vs"], lengths=lengths)
+    assert np.isfinite(got).all()
+    return (np.linalg.norm(got - want, axis=-1) / np.linalg.norm(want, axis=-1)).max()
+
+
+# fp32 sums of up to 2052 weighted terms and fp32 scores below 2^5: a few 1e-6
+# at most; the scales themselves are exact inputs.
+RANGE_BOUND = 1e-5
+
+
+@pytest.mark.parametrize("name", SHAPES)
+def test_tiny_v_scales(o, name):
+    """V scales near the low end of the normal range: all of a sequence's, and
+    those of its first tile (one of them subnormal) before ordinary ones."""
+    rng, p, lengths, page = _problem(o, name, 5)
+    vs = p["vs"]
+    for top in (2.0 ** -100, 2.0 ** -115):
+        p["vs"] = vs * np.float32(top / vs.max())
+        assert _relative_error(_decode(rng, p, lengths, page), p, lengths) <= RANGE_BOUND
+    p["vs"] = vs.copy()
+    p["vs"][:, :, :32] *= np.float32(2.0 ** -115)
+    p["vs"][:, :, 9] = np.float32(2.0 ** -140)
+    assert _relative_error(_decode(rng, p, lengths, page), p, lengths) <= RANGE_BOUND
+
+
+PADDED = [n for n in SHAPES if n != "full_tiles"]
+
+
+@pytest.mark.parametrize("name", PADDED)
+def test_huge_v_scales(o, name):
+    """A V scale of 1.5 * 2^127 at token 0, which has most of the weight, and of
+    2^118 elsewhere, on V rows of -1, 0 and 1 (so that the unnormalised sums of
+    any part of the sequence are in fp32's range)."""
+    rng, p, lengths, page = _problem(o, name, 6)
+    d = p["q"].shape[2]
+    p["q"] = np.abs(p["q"]) + np.float32(0.5)
+    p["k"][:, :, 0] = 127
+    p["ks"][:, :, 0] = 10.0 / (127 * 1.3 * d ** 0.5)
+    p["ks"][:, :, 1:] *= np.float32(1e-3)
+    p["v"] = np.sign(p["v"]).astype(np.int8)
+    p["vs"] = p["vs"] / p["vs"].max() * np.float32(2.0 ** 118)
+    p["vs"][:, :, 0] = np.float32(1.5 * 2.0 ** 127)
+    assert _relative_error(_decode(rng, p, lengths, page), p, lengths) <= RANGE_BOUND
+
+
+@pytest.mark.parametrize("name", PADDED)
+def test_zero_and_non_finite_v_scales(o, name):
+    """Scales of 0 give 0; a NaN scale makes every dim of its sequence and kv
+    head NaN, an infinite one infinite with V's sign, or NaN where V is 0 in
+    that token."""
+    rng, p, lengths, page = _problem(o, name, 7)
+    G = p["q"].shape[1] // p["k"].shape[1]
+    v = p["v"][1, 0, 9] if len(p["q"]) > 1 else p["v"][0, 0, 9]
+    b = 1 if len(p["q"]) > 1 else 0
+    p["vs"][b, 0, 9] = np.inf
+    p["vs"][b, 1, 5] = np.nan
+    if b:
+        p["vs"][0, 0] = 0.0
+    got = _decode(rng, p, lengths, page)
+    heads = got[b, :G]
+    assert np.array_equal(np.isnan(heads), np.broadcast_to(v == 0, heads.shape))
+    assert np.array_equal(np.isposinf(heads), np.broadcast_to(v > 0, heads.shape))
+    assert np.isnan(got[b, G:2 * G]).all()
+    if b:
+        assert (got[0, :G] == 0.0).all()
+        assert np.isfinite(got[2:]).all()
