@@ -106,12 +106,18 @@ __device__ __forceinline__ float next_vref(float vref, float vmax, float& winv, 
     }
 }
 
-// The low half of a PV weight.  PAD: finite where the weight is infinite (an
-// infinite scale), so that the sum of both halves' products is infinite, not NaN.
+// The low half of a PV weight, times kLowScale.  PAD: scaled up by f16's 11
+// bits (its rows are scaled back when the halves are added), so that a weight
+// keeps hi + lo's 22 bits and sign down to 2^-28 of the largest one; unscaled,
+// lo's step of 2^-24 leaves fewer from 2^-17 down (the FMA kernels hold fp32
+// weights of any size).  And finite where the weight is infinite (an infinite
+// scale), so that the sum of both halves' products is infinite, not NaN.
+template <bool PAD>
+constexpr float low_scale() { return PAD ? 2048.0f : 1.0f; }
 template <bool PAD>
 __device__ __forceinline__ _Float16 low_part(float w, _Float16 hi) {
-    const float lo = w - static_cast<float>(hi);
-    return static_cast<_Float16>(PAD ? __builtin_amdgcn_fmed3f(lo, -16.0f, 16.0f) : lo);
+    const float lo = (w - static_cast<float>(hi)) * low_scale<PAD>();
+    return static_cast<_Float16>(PAD ? __builtin_amdgcn_fmed3f(lo, -32768.0f, 32768.0f) : lo);
 }
 
 __device__ __forceinline__ int pack_bytes(const int* b) {
@@ -621,10 +627,11 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
     lsum += __shfl_xor(lsum, 32);
     __syncthreads();  // every wave is done with its V tiles (s_acc reuses them)
     const float fct = vref * (1.0f / weight_scale<PAD>());
+    const float row_fct = lo_row ? fct * (1.0f / low_scale<PAD>()) : fct;
 #pragma unroll
     for (int c = 0; c < NB; c++) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) s_acc[wave][r][16 * c + 4 * g + i] = acc[c][i] * fct;
+        for (int i = 0; i < 4; i++) s_acc[wave][r][16 * c + 4 * g + i] = acc[c][i] * row_fct;
     }
     if (g == 0 && r < G) {
         s_ml[wave][r][0] = m;
@@ -1294,8 +1301,9 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
             // Row r < G (hi part) adds row r + G (lo part): a DPP row shift left by G.
 #pragma unroll
             for (int i = 0; i < 4; i++)
-                o[i] = (acc[c][i] + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc[c][i]),
-                                                                                 0x100 + G, 0xF, 0xF, false))) * unit * sc;
+                o[i] = fmaf(__int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc[c][i]), 0x100 + G, 0xF, 0xF,
+                                                                       false)),
+                            1.0f / low_scale<PAD>(), acc[c][i]) * unit * sc;
             if (writer && (!PAD || 16 * c < d)) {
                 if (complete) {
 #pragma unroll

@@ -141,3 +141,16 @@ def test_zero_and_non_finite_v_scales(o, name):
     if b:
         assert (got[0, :G] == 0.0).all()
         assert np.isfinite(got[2:]).all()
+
+
+@pytest.mark.parametrize("name", PADDED)
+def test_weights_far_below_the_largest_scale(o, name):
+    """One token whose V scale is 2^26 times the others' and whose weight is
+    nothing: the others' weights keep their bits (their products with the
+    scale lie below 2^-26 of the running reference)."""
+    rng, p, lengths, page = _problem(o, name, 8)
+    p["q"] = np.abs(p["q"]) + np.float32(0.5)
+    p["k"][:, :, 7] = -127
+    p["ks"][:, :, 7] = 100.0
+    p["vs"][:, :, 7] = p["vs"].mean() * np.float32(2.0 ** 26)
+    assert _relative_error(_decode(rng, p, lengths, page), p, lengths) <= RANGE_BOUND
