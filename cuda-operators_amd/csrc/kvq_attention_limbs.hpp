@@ -29,7 +29,7 @@
 // * O^T += V^T P^T, six MFMAs per 16-dim block.
 // An input that is not finite, or a product that overflows, leaves NaN or
 // infinity in the wave's state (a limb of it is NaN); the wave then recomputes
-// its queries in fp32 (attention_row).
+// its queries in fp32 (attention_block16).
 //
 // Splits write the (m, l, acc) records that attention_merge combines.  Measured
 // against the kernel on v_mfma_f32_16x16x4_f32 that this one replaced: M = N =
@@ -71,8 +71,83 @@ __device__ __forceinline__ f32x4 mma(const uint4& a, const uint4& b, f32x4 c) {
                                                    0, 0);
 }
 
+// 16 queries from q0 over keys [k0, k1) by one wave on v_mfma_f32_16x16x4_f32:
+// fp32 products in place of the limbs', the same state (o, m and the lane's
+// part of l, relative to the exact running max).  K, V and q come straight from
+// memory, 16 keys at a time; elements past d and rows past k1 or M are zeros.
+// It runs for the waves whose limbs do not hold their values, so it keeps few
+// registers and no loads in flight over a block: 2-3 times the limb kernel's
+// time if every wave takes it (M = N = 4096 d = 128 142 us, and 5920 with one
+// query at a time in FMAs; M = 1000 N = 3001 d = 96 41 us, 1265).
+template <int D>
+__device__ __forceinline__ void attention_block16(const AttnArgs& a, int q0, int k0, int k1, f32x4 (&o)[D / 16], float& m,
+                                                  float& l) {
+    constexpr int NB = D / 16;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int r = lane & 15;
+    const int g = lane >> 4;
+    const int d = a.d;
+    // Row r of 16 rows, dims 16 j + 4 g + [0, 4): one contraction index of four steps.
+    auto piece = [&](buf_rsrc rs, int j) {
+        const int c = 16 * j + 4 * g;
+        float4 x = __builtin_bit_cast(float4, buffer_load16(rs, c < d ? (r * d + c) * 4 : kLimbOob, 0));
+        if (c + 1 >= d) x.y = 0.0f;
+        if (c + 2 >= d) x.z = 0.0f;
+        if (c + 3 >= d) x.w = 0.0f;
+        return x;
+    };
+    const buf_rsrc qr = make_rsrc(a.q + static_cast<size_t>(q0) * d, static_cast<unsigned>(min(16, a.M - q0)) * d * 4u);
+#pragma unroll
+    for (int c = 0; c < NB; c++) o[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    m = -INFINITY;
+    l = 0.0f;
+#pragma unroll 1
+    for (int t = k0; t < k1; t += 16) {
+        const unsigned bytes = static_cast<unsigned>(min(16, k1 - t)) * d * 4u;
+        const buf_rsrc kr = make_rsrc(a.k + static_cast<size_t>(t) * d, bytes);
+        const buf_rsrc vr = make_rsrc(a.v + static_cast<size_t>(t) * d, bytes);
+        f32x4 s = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            const float4 x = piece(kr, j);
+            const float4 y = piece(qr, j);
+            s = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, y.x * a.scale_log2, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, y.y * a.scale_log2, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_16x16x4f32(x.z, y.z * a.scale_log2, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w, y.w * a.scale_log2, s, 0, 0, 0);
+        }
+        // s[i]: score of key t + 4 g + i for query q0 + r.
+#pragma unroll
+        for (int i = 0; i < 4; i++) s[i] = t + 4 * g + i < k1 ? s[i] : -INFINITY;
+        float mt = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+        mt = fmaxf(mt, __shfl_xor(mt, 16));
+        mt = fmaxf(mt, __shfl_xor(mt, 32));
+        const float mn = fmaxf(m, mt);
+        const float ms = mn == -INFINITY ? 0.0f : mn;
+        const float alpha = fast_exp2(m - ms);
+        m = mn;
+        l *= alpha;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            s[i] = fast_exp2(s[i] - ms);
+            l += s[i];
+        }
+#pragma unroll
+        for (int c = 0; c < NB; c++) {
+            o[c] *= alpha;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int off = 16 * c + r < d ? ((4 * g + i) * d + 16 * c + r) * 4 : kLimbOob;
+                const float v = __int_as_float(buffer_load4(vr, off, 0));
+                o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, s[i], o[c], 0, 0, 0);
+            }
+        }
+    }
+}
+
 template <int D, int W, int QB, int BUFS>
-__global__ __launch_bounds__(W* kWave) void attention_limbs(const AttnArgs a) {
+__global__ __launch_bounds__(W* kWave) __attribute__((amdgpu_waves_per_eu(D <= 32 ? 4 : W / 4))) void attention_limbs(
+    const AttnArgs a) {  // (two workgroups per CU at D = 32, one otherwise)
     static_assert(D % 32 == 0, "whole 32-dim contraction steps");
     constexpr bool kPhased = W == 8 && BUFS == 2;
     constexpr int AK = kLimbKeys;
@@ -84,7 +159,6 @@ __global__ __launch_bounds__(W* kWave) void attention_limbs(const AttnArgs a) {
     __shared__ __align__(16) unsigned short s_kt[BUFS][3 * AK * KS];
     __shared__ __align__(16) unsigned short s_vt[BUFS][3 * D * VS];
     static_assert(sizeof(s_kt) + sizeof(s_vt) <= 160 * 1024, "LDS");
-    static_assert(sizeof(s_kt) >= sizeof(float) * W * D, "attention_row's accumulators");
 
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -382,35 +456,28 @@ __global__ __launch_bounds__(W* kWave) void attention_limbs(const AttnArgs a) {
         }
     }
 
-    // The normalised output (one split) or the partial record of (split, query).
-    const bool whole = a.splits == 1;
-    const int ps = attention_record_dim(d);
     float bad = 0.0f;
 #pragma unroll
     for (int b = 0; b < QB; b++) {
-        l[b] += __shfl_xor(l[b], 16);
-        l[b] += __shfl_xor(l[b], 32);
         bad = fmaf(l[b], 0.0f, bad);
 #pragma unroll
         for (int c = 0; c < NB; c++)
 #pragma unroll
             for (int i = 0; i < 4; i++) bad = fmaf(o[b][c][i], 0.0f, bad);
     }
-    if (__builtin_amdgcn_ballot_w64(!(bad == 0.0f)) != 0) {
-        float* const acc = reinterpret_cast<float*>(s_kt) + wave * D;  // K tiles: every wave's last read is past
-        for (int q = q0; q < min(q0 + 16 * QB, a.M); q++) {
-            float mq, lq;
-            attention_row(a, q, k0, k1, acc, mq, lq);
-            float* const row = whole ? a.out + static_cast<size_t>(q) * d
-                                     : a.part_acc + (static_cast<size_t>(split) * a.M + q) * ps;
-            for (int j = lane; j < d; j += kWave) row[j] = whole ? acc[j] / lq : acc[j];
-            if (!whole && lane == 0)
-                *reinterpret_cast<float2*>(a.part_ml + (static_cast<size_t>(split) * a.M + q) * 2) = make_float2(mq, lq);
-        }
-        return;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(bad == 0.0f)) != 0, 0)) {
+#pragma unroll
+        for (int b = 0; b < QB; b++)
+            if (q0 + 16 * b < a.M) attention_block16<D>(a, q0 + 16 * b, k0, k1, o[b], m[b], l[b]);
     }
+
+    // The normalised output (one split) or the partial record of (split, query).
+    const bool whole = a.splits == 1;
+    const int ps = attention_record_dim(d);
 #pragma unroll
     for (int b = 0; b < QB; b++) {
+        l[b] += __shfl_xor(l[b], 16);
+        l[b] += __shfl_xor(l[b], 32);
         const int q = q0 + 16 * b + r;
         if (q >= a.M) continue;
         const float inv = whole ? 1.0f / l[b] : 1.0f;

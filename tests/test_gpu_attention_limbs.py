@@ -78,7 +78,7 @@ def test_rescaled_maximum(M, N, d):
 
 @pytest.mark.parametrize("splits", [1, None])
 def test_overflow_and_non_finite(splits):
-    """Values whose limbs overflow or are not finite take the fp32 rows: a key
+    """Values whose limbs overflow or are not finite take fp32 products: a key
     whose score is -inf has weight 0, an infinite V element stays in its column."""
     q, k, v = _problem(90, 300, 96, 11)
     q = np.abs(q) + np.float32(1.0)
@@ -93,3 +93,49 @@ def test_overflow_and_non_finite(splits):
     out, _ = _run(q, k, vv, splits)
     rest = np.arange(96) != 5
     assert np.isposinf(out[:, 5]).all() and np.abs(out - _exact(q, k, v))[:, rest].max() <= BOUND
+
+
+@pytest.mark.parametrize("d", [1, 31, 32, 50, 64, 96, 127, 128, 160, 192, 255, 256])
+@pytest.mark.parametrize("M,N,splits", [(70, 95, 1), (300, 950, None), (1089, 2100, 2), (2100, 2050, None)])
+def test_fp32_products_at_tile_edges(d, M, N, splits):
+    """Every wave on the fp32 products (an infinite V element and a key of -inf
+    scores in the keys of each split): each block size, rows past M, keys past
+    N, dims past d."""
+    q, k, v = _problem(M, N, d, M + N + d)
+    q = np.abs(q) + np.float32(0.5)
+    out, info = _run(q, k, v, splits)
+    dead = np.arange(info.chunk // 2, N, max(16, info.chunk // 3))
+    k[dead] = -np.inf
+    v[dead[:-1]] = 0.0
+    ref = _exact(q, np.delete(k, dead, 0), np.delete(v, dead, 0))
+    out, _ = _run(q, k, v, splits)
+    assert np.abs(out - ref).max() <= BOUND
+    v[N // 3, d // 2] = -np.inf
+    out, _ = _run(q, k, v, splits)
+    rest = np.arange(d) != d // 2
+    assert (out[:, d // 2] == -np.inf).all() if N // 3 not in dead else np.isnan(out[:, d // 2]).all()
+    assert rest.sum() == 0 or np.abs(out - ref)[:, rest].max() <= BOUND
+
+
+def test_non_finite_values_cost_a_few_times_more_at_most():
+    """One infinity in V sends every wave to the fp32 products, which take 2-3
+    times as long as the limbs (one query at a time they took 100 times)."""
+    q, k, v = (torch.randn((4096, 128), device="cuda") for _ in range(3))
+    out = torch.empty_like(q)
+
+    def best(v):
+        t = []
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            kvq.attention_online(q, k, v, out)
+            a.record()
+            for _ in range(5):
+                kvq.attention_online(q, k, v, out)
+            b.record()
+            torch.cuda.synchronize()
+            t.append(a.elapsed_time(b))
+        return min(t)
+
+    finite = best(v)
+    v[2048, 3] = np.inf
+    assert best(v) < 12 * finite
