@@ -28,8 +28,10 @@
 //   needs no data movement, only its limb split.
 // * O^T += V^T P^T, six MFMAs per 16-dim block.
 // An input that is not finite, or a product that overflows, leaves NaN or
-// infinity in the wave's state (a limb of it is NaN); the wave then recomputes
-// its queries in fp32 (attention_block16).
+// infinity in the wave's state (a limb of it is NaN), and values below 2^-110
+// have fewer bits than 24 (bf16's subnormals end at 2^-133); a wave that sees the
+// first, or rows where the second counts (kLimbMin), recomputes its queries in
+// fp32 (attention_block16).
 //
 // Splits write the (m, l, acc) records that attention_merge combines.  Measured
 // against the kernel on v_mfma_f32_16x16x4_f32 that this one replaced: M = N =
@@ -52,6 +54,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kLimbKeys = kAttnLimbTile;  // keys per LDS tile
 constexpr float kLazyMax = 8.0f;          // log2 units a score may pass the softmax reference by
+constexpr float kLimbMin = 0x1p-60f;      // rows of q, and outputs, all below it take fp32 products
 constexpr int kLimbOob = INT_MIN;         // byte offset of a load that reads zeros (past every resource)
 
 // The limbs of a pair of floats, packed: h, m and l of x in the low halves, of y in the high.
@@ -72,8 +75,8 @@ __device__ __forceinline__ f32x4 mma(const uint4& a, const uint4& b, f32x4 c) {
 }
 
 // 16 queries from q0 over keys [k0, k1) by one wave on v_mfma_f32_16x16x4_f32:
-// fp32 products in place of the limbs', the same state (o, m and the lane's
-// part of l, relative to the exact running max).  K, V and q come straight from
+// fp32 products in place of the limbs', the same state (o, m and the whole l,
+// relative to the exact running max).  K, V and q come straight from
 // memory, 16 keys at a time; elements past d and rows past k1 or M are zeros.
 // It runs for the waves whose limbs do not hold their values, so it keeps few
 // registers and no loads in flight over a block: 2-3 times the limb kernel's
@@ -143,6 +146,8 @@ __device__ __forceinline__ void attention_block16(const AttnArgs& a, int q0, int
             }
         }
     }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
 }
 
 template <int D, int W, int QB, int BUFS>
@@ -456,16 +461,38 @@ __global__ __launch_bounds__(W* kWave) __attribute__((amdgpu_waves_per_eu(D <= 3
         }
     }
 
-    float bad = 0.0f;
+    // What the limbs cannot hold: NaN or infinity in the state, and values below
+    // 2^-110, of which up to 2^-126 can be lost (a limb under bf16's subnormals).
+    // That is nothing in an output row whose largest element is above kLimbMin
+    // (weights sum to 1 or more), and nothing in the scores of a q row whose
+    // largest is above kLimbMin and not above its reciprocal (or 0).  A row is
+    // spread over four lane groups, whose ballots are folded.
+    unsigned long long bad = 0;
+    auto none = [](bool x) {  // rows for which no group has x, in the low 16 bits
+        const unsigned long long y = __builtin_amdgcn_ballot_w64(x);
+        return ~(y | y >> 16 | y >> 32 | y >> 48) & 0xffff;
+    };
 #pragma unroll
     for (int b = 0; b < QB; b++) {
-        bad = fmaf(l[b], 0.0f, bad);
+        float top = 0.0f;
 #pragma unroll
         for (int c = 0; c < NB; c++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) bad = fmaf(o[b][c][i], 0.0f, bad);
+            for (int i = 0; i < 4; i++) top = max_or_nan(top, fabsf(o[b][c][i]));
+        typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+        u16x2 qt = {0, 0};  // high limbs' magnitudes
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (const unsigned x : {qh[b][s].x, qh[b][s].y, qh[b][s].z, qh[b][s].w})
+                qt = __builtin_elementwise_max(qt, __builtin_bit_cast(u16x2, x & 0x7fff7fffu));
+        const float qmax = __uint_as_float(static_cast<unsigned>(max(qt.x, qt.y)) << 16);
+        bad |= __builtin_amdgcn_ballot_w64(!(top < INFINITY && l[b] < INFINITY && qmax <= 1.0f / kLimbMin)) |
+               none(top >= kLimbMin) | (none(qmax >= kLimbMin) & ~none(qmax != 0.0f));
+        l[b] += __shfl_xor(l[b], 16);
+        l[b] += __shfl_xor(l[b], 32);
     }
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(bad == 0.0f)) != 0, 0)) {
+    if (__builtin_expect(bad != 0, 0)) {
 #pragma unroll
         for (int b = 0; b < QB; b++)
             if (q0 + 16 * b < a.M) attention_block16<D>(a, q0 + 16 * b, k0, k1, o[b], m[b], l[b]);
@@ -476,8 +503,6 @@ __global__ __launch_bounds__(W* kWave) __attribute__((amdgpu_waves_per_eu(D <= 3
     const int ps = attention_record_dim(d);
 #pragma unroll
     for (int b = 0; b < QB; b++) {
-        l[b] += __shfl_xor(l[b], 16);
-        l[b] += __shfl_xor(l[b], 32);
         const int q = q0 + 16 * b + r;
         if (q >= a.M) continue;
         const float inv = whole ? 1.0f / l[b] : 1.0f;

@@ -77,9 +77,6 @@ __device__ __forceinline__ f16x8 i8x8_to_f16(i32x2 v) {
     return f16x8{h0.x, h0.y, h1.x, h1.y, h2.x, h2.y, h3.x, h3.y};
 }
 
-// The larger of two floats, NaN if either is (v_maximum3_f32).
-__device__ __forceinline__ float max_or_nan(float x, float y) { return __builtin_elementwise_maximum(x, y); }
-
 // PV weights are w = p * v_scale * weight_scale / vref, |w| <= 2^15.  vref after
 // a tile whose largest |v_scale|, or kVrefMin if that is larger, is vmax; also
 // winv = weight_scale / vref and ratio = old vref / new.  With the floor winv stays finite for V rows of any size (with the reciprocal of a smaller

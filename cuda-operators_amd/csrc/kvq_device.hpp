@@ -108,6 +108,9 @@ __device__ __forceinline__ float wave_max(float x) {
     return x;
 }
 
+// The larger of two floats, NaN if either is (v_maximum3_f32).
+__device__ __forceinline__ float max_or_nan(float x, float y) { return __builtin_elementwise_maximum(x, y); }
+
 // Signed byte b of a dword as float: one v_cvt_f32_i32 with an SDWA
 // sign-extended byte select on gfx950.
 __device__ __forceinline__ float sbyte(int w, int b) {

@@ -139,3 +139,25 @@ def test_non_finite_values_cost_a_few_times_more_at_most():
     finite = best(v)
     v[2048, 3] = np.inf
     assert best(v) < 12 * finite
+
+
+@pytest.mark.parametrize("M,N,d", [(70, 95, 96), (300, 950, 50), (1089, 2100, 128)])
+@pytest.mark.parametrize("splits", [1, None])
+def test_values_below_the_limbs_range(M, N, d, splits):
+    """Values whose third limb is below bf16's subnormals keep fp32's precision:
+    V rows of 2^-118, and tiny q against huge K and the reverse.  Error over the
+    output's norm; BOUND's scores, V of one magnitude."""
+    q, k, v = _problem(M, N, d, M)
+
+    def check(q, k, v, what):
+        out, _ = _run(q, k, v, splits)
+        want = _exact(q, k, v)
+        err = np.linalg.norm(out - want, axis=1) / np.linalg.norm(want, axis=1)
+        assert err.max() <= BOUND, (what, err.max())
+
+    check(q, k, (v * 2.0 ** -118).astype(np.float32), "V")
+    check((q * 2.0 ** -118).astype(np.float32), (k * 2.0 ** 118).astype(np.float32), v, "q")
+    check((q * 2.0 ** 118).astype(np.float32), (k * 2.0 ** -118).astype(np.float32), v, "K")
+    q[M // 2] *= np.float32(2.0 ** -118)  # one row of many
+    q[3] = 0.0
+    check(q, k, v, "one row")
