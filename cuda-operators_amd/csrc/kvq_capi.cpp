@@ -686,8 +686,17 @@ bool attention_args_ok(int M, int N, int d, const void* q, const void* k, const 
     return N <= INT_MAX - 1024 && M <= INT_MAX - 1024;
 }
 
-// owned: the workspace is the library's.  A caller's own workspace was never
-// needed at head dims without a few-query kernel, so there it stays unsplit.
+// Calls that need no memory, whatever plan is the fastest: head dims without a
+// few-query kernel, and M whose 128-query blocks fill the GPU alone (256
+// workgroups, below d = 128 512).  Programs may make them without a workspace,
+// or under capture without an eager call before.
+bool attention_needed_no_memory(int M, int d) {
+    return !kvq::attention_rows_dim(d) || (static_cast<long long>(M) + 127) / 128 >= (d >= 128 ? 256 : 512);
+}
+
+// owned: the workspace is the library's.  With a caller's own, the calls above
+// run unsplit (those M in 128-query blocks; in the library's workspace two
+// splits of 256-query blocks take M = 32768 N = 8192 d = 128 570 us, against 665).
 AttnPlan attention_plan(int M, int N, int d, bool aligned, int requested, bool owned) {
     AttnPlan p;
     p.tuned = d <= kvq::kAttnLimbMaxDim && aligned;
@@ -757,9 +766,11 @@ AttnPlan attention_plan(int M, int N, int d, bool aligned, int requested, bool o
     // 52.2 / 52.8, d = 64 37.0 / 34.4, M = N = 8192 d = 64 (128) 95.9 / 87.5.
     const long long work = (static_cast<long long>(M) + 63) / 64 *
                            ((static_cast<long long>(N) + kvq::kAttnLimbTile - 1) / kvq::kAttnLimbTile);
-    p.qblock = M <= 64 || work < 7 * 256                                      ? 64
-               : M > 512 && d <= 128 && work >= (d <= 64 ? 32 : 64) * 256LL ? 256
-                                                                              : 128;
+    const bool rows_dim = kvq::attention_rows_dim(d);
+    const bool unsplit = !owned && attention_needed_no_memory(M, d) && (requested == 0 || !rows_dim);
+    p.qblock = M <= 64 || work < 7 * 256                                                                 ? 64
+               : M > 512 && d <= 128 && work >= (d <= 64 ? 32 : 64) * 256LL && !(unsplit && rows_dim) ? 256
+                                                                                                         : 128;
     // Key splits for one round of workgroups (one per CU; two at d <= 32: M = N
     // = 8192 70.3 us with one, 61.7 with two), never a few more than a round
     // (M = 700, N = 9000, d = 80 in 64-query blocks: 264 workgroups 41.9 us).
@@ -768,7 +779,7 @@ AttnPlan attention_plan(int M, int N, int d, bool aligned, int requested, bool o
     const long long target = d <= 32 ? 512 : 256;
     const long long qblocks = (static_cast<long long>(M) + p.qblock - 1) / p.qblock;
     long long want = requested > 0 ? requested : std::max(1LL, target / qblocks);
-    if (!owned && !kvq::attention_rows_dim(d)) want = 1;
+    if (unsplit) want = 1;
     want = std::max(1LL, std::min({want, tiles, static_cast<long long>(kvq::attention_max_splits(d))}));
     // The merge runs up to 64 lanes per 16-byte output column, indexed in int.
     if (static_cast<long long>(M) * (kvq::attention_record_dim(d) / 4) * 64 >= INT_MAX) want = 1;

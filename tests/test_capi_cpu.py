@@ -488,6 +488,18 @@ def test_attention_plan_routes_misaligned_to_generic(L):
                 assert L.kvq_attention_workspace_size(ctypes.byref(p)) == 0
 
 
+@pytest.mark.parametrize("d,M", [(128, 32641), (128, 32768), (32, 65409), (32, 65536), (256, 32700), (64, 65500)])
+def test_attention_plan_needs_no_memory_once_128_query_blocks_fill_the_gpu(L, d, M):
+    """One round of 128-query blocks (256, or 512 below d = 128) runs unsplit:
+    callers without a workspace may make these calls."""
+    A = 1 << 20
+    for N in (64, 1100, 5000, 65536):
+        p = kvq.AttentionParams(M, N, d, A, A, A, A, 0.0, 0)
+        info = kvq.attention_plan(p)
+        assert (info.kernel, info.splits, info.workspace_bytes) == (kvq.KERNEL_ATTENTION_MFMA, 1, 0)
+        assert L.kvq_attention_workspace_size(ctypes.byref(p)) == 0
+
+
 def _diagnostics_with(env_updates):
     env = dict(os.environ)
     env.pop("KVQ_DEBUG_SYNC", None)
