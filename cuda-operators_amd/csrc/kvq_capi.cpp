@@ -829,8 +829,12 @@ hipError_t attention_run(int M, int N, int d, const float* q, const float* k, co
 // captured from an earlier call on this stream still writes to it on every
 // replay (so the retired bytes stay below the live ones).  Growing needs
 // hipMalloc, which a capturing stream does not allow: run one eager call of
-// the largest problem before capturing.  As for `solve`, `launch(ptr)` is
-// enqueued under the lock.
+// the largest problem before capturing.  Of the calls that need no memory
+// (attention_needed_no_memory) a captured one that finds too small a workspace,
+// and an eager one that gets none, run unsplit instead.
+// The allocation is made in relaxed capture mode, so that it does not end
+// another thread's capture.  As for `solve`, `launch(ptr)` is enqueued under
+// the lock.
 struct AttnWorkspaceKey {
     int device;
     hipStream_t stream;
@@ -842,8 +846,19 @@ std::mutex g_attn_ws_mutex;
 std::map<AttnWorkspaceKey, SolveWorkspace> g_attn_ws;
 std::vector<void*> g_attn_retired;
 
-template <class Launch>
-hipError_t with_attention_workspace(size_t need, hipStream_t stream, Launch&& launch) {
+hipError_t malloc_relaxed(void** ptr, size_t bytes) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    hipError_t err = hipThreadExchangeStreamCaptureMode(&mode);
+    if (err != hipSuccess) return err;
+    err = hipMalloc(ptr, bytes);
+    const hipError_t back = hipThreadExchangeStreamCaptureMode(&mode);
+    return err != hipSuccess ? err : back;
+}
+
+// unsplit: the call without a workspace, where it must not fail for want of one.
+template <class Launch, class Unsplit>
+hipError_t with_attention_workspace(size_t need, hipStream_t stream, Launch&& launch, bool may_unsplit,
+                                    Unsplit&& unsplit) {
     if (need == 0) return launch(nullptr);
     int dev = 0;
     hipError_t err = hipGetDevice(&dev);
@@ -851,10 +866,18 @@ hipError_t with_attention_workspace(size_t need, hipStream_t stream, Launch&& la
     std::lock_guard<std::mutex> lock(g_attn_ws_mutex);
     SolveWorkspace& w = g_attn_ws[AttnWorkspaceKey{dev, stream}];
     if (w.bytes < need) {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        err = hipStreamIsCapturing(stream, &st);
+        if (err != hipSuccess) return err;
+        if (st != hipStreamCaptureStatusNone && may_unsplit) return unsplit();
         const size_t bytes = round_up(std::max(need, 2 * w.bytes), 1 << 20);
         void* ptr = nullptr;
-        err = hipMalloc(&ptr, bytes);
-        if (err != hipSuccess) return err;
+        err = st == hipStreamCaptureStatusNone ? malloc_relaxed(&ptr, bytes) : hipMalloc(&ptr, bytes);
+        if (err != hipSuccess) {
+            if (!may_unsplit) return err;
+            (void)hipGetLastError();  // the launch below reports its own status
+            return unsplit();
+        }
         if (w.ptr) g_attn_retired.push_back(w.ptr);  // still referenced by any graph captured before
         w.ptr = ptr;
         w.bytes = bytes;
@@ -1087,11 +1110,15 @@ hipError_t kvq_prefill_quantize_launch(const kvq_prefill_params* p, hipStream_t 
 hipError_t attention_online_launch(const float* Q, const float* K, const float* V, float* output, int M, int N,
                                    int d, hipStream_t stream) {
     if (!attention_args_ok(M, N, d, Q, K, V, output)) return hipErrorInvalidValue;
-    const AttnPlan p = attention_plan(M, N, d, attention_aligned(Q, K, V, output), 0, true);
+    const bool aligned = attention_aligned(Q, K, V, output);
+    const AttnPlan p = attention_plan(M, N, d, aligned, 0, true);
+    auto run = [&](const AttnPlan& plan, void* ws) {
+        return attention_run(M, N, d, Q, K, V, output, 1.0f / sqrtf(static_cast<float>(d)), plan, ws, stream);
+    };
     return checked_call(stream, [&] {
-        return with_attention_workspace(p.bytes(), stream, [&](void* ws) {
-            return attention_run(M, N, d, Q, K, V, output, 1.0f / sqrtf(static_cast<float>(d)), p, ws, stream);
-        });
+        return with_attention_workspace(
+            p.bytes(), stream, [&](void* ws) { return run(p, ws); }, attention_needed_no_memory(M, d),
+            [&] { return run(attention_plan(M, N, d, aligned, 0, false), nullptr); });
     });
 }
 

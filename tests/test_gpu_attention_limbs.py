@@ -161,3 +161,31 @@ def test_values_below_the_limbs_range(M, N, d, splits):
     q[M // 2] *= np.float32(2.0 ** -118)  # one row of many
     q[3] = 0.0
     check(q, k, v, "one row")
+
+
+@pytest.mark.parametrize("M,N,d", [(300, 950, 96), (70, 9000, 50), (32700, 1100, 128)])
+def test_capture_without_an_eager_call_before(M, N, d):
+    """Calls that ran without memory before they were split can be captured on
+    a stream that has none yet (they run unsplit there), with eager calls on
+    the same stream between the replays."""
+    q, k, v = (up(x) for x in _problem(M, N, d, 21))
+    assert kvq.attention_plan(kvq.attention_params(q, k, v, q)).kernel == kvq.KERNEL_ATTENTION_MFMA
+    rows = np.random.default_rng(2).permutation(M)[:64]
+    out, eager = torch.empty_like(q), torch.empty_like(q)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        kvq.attention_online(q, k, v, out)
+    for rep in range(3):
+        q.copy_(up(_problem(M, 1, d, 30 + rep)[0]))
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s):
+            kvq.attention_online(q, k, v, eager)
+        s.synchronize()
+        want = _exact(down(q)[rows], down(k), down(v))
+        for got in (out, eager):
+            assert np.abs(down(got)[rows] - want).max() <= BOUND, rep
