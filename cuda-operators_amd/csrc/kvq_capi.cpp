@@ -230,7 +230,6 @@ DecodePlan make_plan(int B, int Hq, int Hkv, int d, int max_len, bool aligned, b
                (padding || kvq::fast_padded_dim(d) == d)) {
         p.kernel = kvq::Kernel::Valu;
         p.sg = sg_v;
-        p.padded = kvq::fast_padded_dim(d) != d;
         tile = kvq::fast_tile_tokens(d, sg_v);
     } else {
         p.kernel = kvq::Kernel::Generic;
@@ -493,8 +492,8 @@ hipError_t with_solve_workspace(size_t need, Launch&& launch) {
 kvq_plan_info decode_info(const DecodePlan& p) {
     kvq_plan_info r{};
     r.kernel = p.kernel == kvq::Kernel::Mfma   ? KVQ_KERNEL_DECODE_MFMA
-               : p.kernel == kvq::Kernel::Valu && !p.padded ? KVQ_KERNEL_DECODE_VALU
-                                                            : KVQ_KERNEL_DECODE_GENERIC;
+               : p.kernel == kvq::Kernel::Valu ? KVQ_KERNEL_DECODE_VALU
+                                               : KVQ_KERNEL_DECODE_GENERIC;
     r.heads_per_group = p.sg;
     r.split_plan = p.flat           ? KVQ_SPLITS_TILES
                    : p.fit || p.lpt ? KVQ_SPLITS_IN_KERNEL

@@ -111,15 +111,14 @@ constexpr int kSizeClasses = 64;
 // Which decode kernel a plan runs.
 enum class Kernel {
     Generic,  // any head dim / alignment (decode_generic)
-    Valu,     // decode_fast: d in {32,64,128,256}, per-lane FMAs
-    Mfma,     // decode_mfma: d a multiple of 16 up to 128, up to 8 query heads per kv head group
+    Valu,     // decode_fast: d = 32 and multiples of 16 from 48 to 256, per-lane FMAs
+    Mfma,     // decode_mfma: d a multiple of 16 from 48 to 128, up to 8 query heads per kv head group
 };
 
 // Launch plan chosen on the host.
 struct DecodePlan {
     Kernel kernel;
     bool fast;       // a tuned kernel (Valu or Mfma): 16-byte aligned rows
-    bool padded;     // Kernel::Valu at a head dim that its lanes pad
     int sg;          // query heads per workgroup (tuned kernels)
     int tile;        // tokens one workgroup iteration covers (tuned kernels; 0: generic)
     int nsg;         // G / sg, rounded up

@@ -320,9 +320,9 @@ const char* kvq_version(void);
  * may be any values with the alignment of the real ones.  They report what
  * the matching launch would do. */
 
-#define KVQ_KERNEL_DECODE_GENERIC 0   /* decode_generic: any head dim or alignment; or, at aligned
-                                         multiples of 16, decode_fast with padded lanes */
-#define KVQ_KERNEL_DECODE_VALU 1      /* decode_fast: per-lane FMAs */
+#define KVQ_KERNEL_DECODE_GENERIC 0   /* decode_generic: any head dim or alignment */
+#define KVQ_KERNEL_DECODE_VALU 1      /* decode_fast: per-lane FMAs; head dim 32 and multiples of 16
+                                         from 48 to 256 (between the powers of two with padded lanes) */
 #define KVQ_KERNEL_DECODE_MFMA 2      /* decode_mfma: grouped-query heads on matrix cores */
 #define KVQ_KERNEL_ATTENTION_MFMA 3   /* attention_limbs: query blocks on matrix cores, d <= 256 */
 #define KVQ_KERNEL_ATTENTION_ROWS 4   /* attention_rows: up to 8 queries per workgroup */

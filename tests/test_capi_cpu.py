@@ -462,7 +462,12 @@ def test_decode_plan_kernels(L):
     i = plan(513, 64, 8, 128, 4096, lengths=A)
     assert (i.kernel, i.heads_per_group, i.split_plan) == (kvq.KERNEL_DECODE_MFMA, 8, kvq.SPLITS_SCHEDULE)
     assert plan(1, 8, 8, 64, 1024).splits == 1                                   # cfg0
-    assert plan(1, 8, 8, 96, 1024).kernel == kvq.KERNEL_DECODE_GENERIC
+    for d in (48, 80, 96, 112, 144, 192, 240):  # padded lanes
+        i = plan(1, 8, 8, d, 1024)
+        assert i.kernel == kvq.KERNEL_DECODE_VALU and i.tile_tokens > 0
+    for d in (16, 40, 100, 272):
+        i = plan(1, 8, 8, d, 1024)
+        assert (i.kernel, i.heads_per_group, i.tile_tokens) == (kvq.KERNEL_DECODE_GENERIC, 1, 0)
     assert plan(1, 8, 8, 128, 1024, misalign=4).kernel == kvq.KERNEL_DECODE_GENERIC
     assert plan(1, 4, 4, 128, 8192, splits=8).splits == 8
 

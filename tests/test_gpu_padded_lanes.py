@@ -41,6 +41,9 @@ def test_padded_lanes(o, G, d, B, cap, ragged, page):
         lengths[:4] = [cap, 1, 31, 33]
     p = make_problem(rng, B, Hkv * G, Hkv, cap, d, o.quantize_rows, lengths=lengths)
     L = lengths if ragged else np.full(B, cap, np.int32)
+    prm = kvq.DecodeParams(B, Hkv * G, Hkv, d, cap, cap, 4096 if ragged else None, *[4096] * 6, 0.0, 0, None, None)
+    info = kvq.decode_plan(prm)
+    assert info.kernel == kvq.KERNEL_DECODE_VALU
     want0 = o.decode_f32(p["q"], p["k"], p["v"], p["ks"], p["vs"], lengths=L)
     got = _gpu.decode(p["q"], p["k"], p["v"], p["ks"], p["vs"], lengths=lengths, max_seq_len=cap)[0]
     assert_close(got, want0, what=f"no append G={G} d={d} B={B}")
@@ -51,6 +54,9 @@ def test_padded_lanes(o, G, d, B, cap, ragged, page):
     if page:
         kp, vp, ksp, vsp, table = to_pages(rng, p["k"], p["v"], p["ks"], p["vs"], lengths, page)
         paged = paged_decode(p["q"], kp, vp, ksp, vsp, table, lengths, k_new=kn, v_new=vn)
+        whole_tiles = page % (info.tile_tokens // 8) == 0  # a wave tile of 8 waves' tokens lies in one page
+        assert kvq.paged_decode_plan(paged[5].params).kernel == (kvq.KERNEL_DECODE_VALU if whole_tiles else
+                                                                  kvq.KERNEL_DECODE_GENERIC)
     o.append(kn, vn, p["k"], p["v"], p["ks"], p["vs"], positions=L - 1)
     assert np.array_equal(gk, p["k"]) and np.array_equal(gv, p["v"])
     assert np.array_equal(_bits(gks), _bits(p["ks"])) and np.array_equal(_bits(gvs), _bits(p["vs"]))
@@ -65,6 +71,7 @@ def test_padded_lanes(o, G, d, B, cap, ragged, page):
 def test_padded_lanes_reference_abi(o, H, N, d):
     rng = np.random.default_rng(N + d)
     Q, K, V, ks, vs = _gpu.reference_problem(H, N, d, rng)
+    assert kvq.reference_plan(H, N, d).kernel == kvq.KERNEL_DECODE_VALU
     want = o.head_f32(Q, K, V, ks, vs)
     for entry in ("solve", "split", "simple"):
         assert_close(_run(entry, Q, K, V, ks, vs), want, what=f"{entry} H{H} N{N} d{d}")
