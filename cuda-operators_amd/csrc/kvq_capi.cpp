@@ -693,9 +693,10 @@ bool attention_needed_no_memory(int M, int d) {
     return !kvq::attention_rows_dim(d) || (static_cast<long long>(M) + 127) / 128 >= (d >= 128 ? 256 : 512);
 }
 
-// owned: the workspace is the library's.  With a caller's own, the calls above
-// run unsplit (those M in 128-query blocks; in the library's workspace two
-// splits of 256-query blocks take M = 32768 N = 8192 d = 128 570 us, against 665).
+// owned: the workspace is the library's.  With a caller's own, those calls run
+// unsplit unless splits are requested, and those M in 128-query blocks (in the
+// library's workspace two splits of 256-query blocks take M = 32768 N = 8192
+// d = 128 570 us, against 665).
 AttnPlan attention_plan(int M, int N, int d, bool aligned, int requested, bool owned) {
     AttnPlan p;
     p.tuned = d <= kvq::kAttnLimbMaxDim && aligned;
@@ -765,11 +766,11 @@ AttnPlan attention_plan(int M, int N, int d, bool aligned, int requested, bool o
     // 52.2 / 52.8, d = 64 37.0 / 34.4, M = N = 8192 d = 64 (128) 95.9 / 87.5.
     const long long work = (static_cast<long long>(M) + 63) / 64 *
                            ((static_cast<long long>(N) + kvq::kAttnLimbTile - 1) / kvq::kAttnLimbTile);
-    const bool rows_dim = kvq::attention_rows_dim(d);
-    const bool unsplit = !owned && attention_needed_no_memory(M, d) && (requested == 0 || !rows_dim);
-    p.qblock = M <= 64 || work < 7 * 256                                                                 ? 64
-               : M > 512 && d <= 128 && work >= (d <= 64 ? 32 : 64) * 256LL && !(unsplit && rows_dim) ? 256
-                                                                                                         : 128;
+    const bool unsplit = !owned && requested == 0 && attention_needed_no_memory(M, d);
+    const bool wide = !(unsplit && kvq::attention_rows_dim(d));
+    p.qblock = M <= 64 || work < 7 * 256                                              ? 64
+               : M > 512 && d <= 128 && work >= (d <= 64 ? 32 : 64) * 256LL && wide ? 256
+                                                                                      : 128;
     // Key splits for one round of workgroups (one per CU; two at d <= 32: M = N
     // = 8192 70.3 us with one, 61.7 with two), never a few more than a round
     // (M = 700, N = 9000, d = 80 in 64-query blocks: 264 workgroups 41.9 us).
@@ -1117,7 +1118,7 @@ hipError_t attention_online_launch(const float* Q, const float* K, const float* 
     return checked_call(stream, [&] {
         return with_attention_workspace(
             p.bytes(), stream, [&](void* ws) { return run(p, ws); }, attention_needed_no_memory(M, d),
-            [&] { return run(attention_plan(M, N, d, aligned, 0, false), nullptr); });
+            [&] { return run(attention_plan(M, N, d, aligned, kvq::attention_rows_dim(d) ? 0 : 1, false), nullptr); });
     });
 }
 
@@ -1131,8 +1132,11 @@ hipError_t kvq_attention_launch(const kvq_attention_params* p, void* workspace, 
                                 hipStream_t stream) {
     if (!p || !attention_args_ok(p->M, p->N, p->d, p->q, p->k, p->v, p->out) || p->num_splits < 0)
         return hipErrorInvalidValue;
-    const AttnPlan plan =
-        attention_plan(p->M, p->N, p->d, attention_aligned(p->q, p->k, p->v, p->out), p->num_splits, false);
+    const bool aligned = attention_aligned(p->q, p->k, p->v, p->out);
+    AttnPlan plan = attention_plan(p->M, p->N, p->d, aligned, p->num_splits, false);
+    // Head dims without a few-query kernel need no workspace; split requests use one.
+    if (plan.bytes() > 0 && !workspace && !kvq::attention_rows_dim(p->d))
+        plan = attention_plan(p->M, p->N, p->d, aligned, 1, false);
     if (plan.bytes() > 0 && (!workspace || workspace_bytes < plan.bytes() || !aligned16(workspace)))
         return hipErrorInvalidValue;
     const float scale = p->softmax_scale != 0.0f ? p->softmax_scale : 1.0f / sqrtf(static_cast<float>(p->d));

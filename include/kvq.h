@@ -307,7 +307,8 @@ size_t kvq_attention_workspace_size(const kvq_attention_params* p);
  * ordered (one stream).  hipErrorInvalidValue, before any HIP call, for the
  * checks of attention_online_launch, M or N above INT_MAX - 1024, a negative
  * num_splits, or a workspace too small, NULL or misaligned when one is
- * needed. */
+ * needed.  At head dims other than 32, 64, 128 and 256 the keys are split only
+ * on request, and a request with a NULL workspace runs unsplit. */
 hipError_t kvq_attention_launch(const kvq_attention_params* p, void* workspace, size_t workspace_bytes,
                                 hipStream_t stream);
 
@@ -356,8 +357,11 @@ hipError_t kvq_reference_plan(const float* Q, const int8_t* K_int8, const int8_t
 hipError_t kvq_decode_plan(const kvq_decode_params* p, kvq_plan_info* info);
 /* The plan of kvq_paged_decode_launch for p. */
 hipError_t kvq_paged_decode_plan(const kvq_paged_decode_params* p, kvq_plan_info* info);
-/* The plan of kvq_attention_launch for p (attention_online_launch: p with
- * softmax_scale 0 and num_splits 0). */
+/* The plan of kvq_attention_launch for p and a workspace of that size; also
+ * that of attention_online_launch (p with softmax_scale 0 and num_splits 0),
+ * except that with its own workspace it splits the keys at every head dim up to
+ * 256, and where this plan needs no workspace because 128-query blocks fill the
+ * GPU (32641 queries at d = 128). */
 hipError_t kvq_attention_plan(const kvq_attention_params* p, kvq_plan_info* info);
 
 /* Diagnostic switches in force, read once from the environment:

@@ -505,6 +505,21 @@ def test_attention_plan_needs_no_memory_once_128_query_blocks_fill_the_gpu(L, d,
         assert L.kvq_attention_workspace_size(ctypes.byref(p)) == 0
 
 
+@pytest.mark.parametrize("d", [30, 96, 192])
+def test_attention_split_requests_at_every_head_dim(L, d):
+    """Head dims without a few-query kernel: unsplit and no workspace unless
+    splits are requested; a request's records are (max, sum) and the accumulator
+    in whole 16-byte columns per split and query."""
+    A = 1 << 20
+    for M, N, splits, want in ((1, 65536, 0, 1), (1000, 3001, 0, 1), (70, 9000, 5, 5), (300, 4096, 64, 64), (300, 4000, 1, 1)):
+        p = kvq.AttentionParams(M, N, d, A, A, A, A, 0.0, splits)
+        info = kvq.attention_plan(p)
+        assert (info.kernel, info.splits) == (kvq.KERNEL_ATTENTION_MFMA, want)
+        rows = want * M if want > 1 else 0
+        assert info.workspace_bytes == _ru(rows * 8) + _ru(rows * ((d + 3) // 4 * 16))
+        assert L.kvq_attention_workspace_size(ctypes.byref(p)) == info.workspace_bytes
+
+
 def _diagnostics_with(env_updates):
     env = dict(os.environ)
     env.pop("KVQ_DEBUG_SYNC", None)

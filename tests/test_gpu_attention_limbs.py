@@ -6,6 +6,7 @@ limb products drop terms below 2^-24 of a product and the sums run in fp32, so
 scores of magnitude s (log2 units, s < 40 here) carry absolute errors of a few
 s * 2^-24, which are relative errors of the weights: 40 * 4 * 2^-24 < 1e-5, of
 max|V| < 6."""
+import ctypes
 import math
 
 import numpy as np
@@ -31,8 +32,7 @@ def _exact(q, k, v):
 
 
 def _run(q, k, v, splits=None):
-    """attention_online's own splits, or kvq.attention with a request (which head dims other than 32, 64, 128 and 256
-    run unsplit)."""
+    """attention_online's own splits, or kvq.attention with a request."""
     gq, gk, gv = up(q), up(k), up(v)
     out = _gpu.poisoned(q.shape)
     info = kvq.attention_plan(kvq.attention_params(gq, gk, gv, out, num_splits=splits or 0))
@@ -189,3 +189,26 @@ def test_capture_without_an_eager_call_before(M, N, d):
         want = _exact(down(q)[rows], down(k), down(v))
         for got in (out, eager):
             assert np.abs(down(got)[rows] - want).max() <= BOUND, rep
+
+
+@pytest.mark.parametrize("d", [30, 96, 192])
+@pytest.mark.parametrize("M,N,splits", [(1, 5000, 40), (70, 1000, 3), (300, 950, 1 << 20), (1089, 2100, 2)])
+def test_caller_workspace_splits_and_null(d, M, N, splits):
+    """A caller's own workspace (NaN-filled, the size the query gives) at head
+    dims without a few-query kernel: a split request, and the same with NULL."""
+    q, k, v = _problem(M, N, d, d + M)
+    want = _exact(q, k, v)
+    g = [up(x) for x in (q, k, v)]
+    out = _gpu.poisoned(q.shape)
+    p = kvq.attention_params(*g, out, num_splits=splits)
+    info = kvq.attention_plan(p)
+    assert info.splits > 1 and info.workspace_bytes > 0
+    ws = torch.full((info.workspace_bytes,), 0xFF, dtype=torch.uint8, device="cuda")
+    kvq.attention(*g, out, num_splits=splits, workspace=ws)
+    torch.cuda.synchronize()
+    assert np.abs(down(out) - want).max() <= BOUND
+    assert (ws != 0xFF).any()  # the records were written
+    out.fill_(float("nan"))
+    assert kvq.lib().kvq_attention_launch(ctypes.byref(p), None, 0, torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert np.abs(down(out) - want).max() <= BOUND
