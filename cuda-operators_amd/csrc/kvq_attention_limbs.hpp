@@ -4,8 +4,8 @@
 // for any d up to 256.
 //
 // Every fp32 value x is three bf16 limbs, h = bf16(x), m = bf16(x - h),
-// l = x - h - m: 8 + 8 + 8 significand bits with signs hold all 24, and the
-// differences are exact.  A product keeps the six limb pairs down to 2^-16 of
+// l = x - h - m: 8 + 8 + 8 significand bits with signs hold all 24 of a value
+// from 2^-110 up, and the differences are exact.  A product keeps the six limb pairs down to 2^-16 of
 // it (hh, hm, mh, mm, hl, lh); the dropped ones are below 2^-24, and bf16
 // products are exact in the fp32 accumulators.  Six v_mfma_f32_16x16x32_bf16
 // take 96 cycles where the eight v_mfma_f32_16x16x4_f32 of the same contraction
@@ -39,7 +39,7 @@
 // 93.8 -> 60.2 us, M = N = 1024 d = 128 16.6 -> 14.8 us; and against
 // attention_generic, M = 1000 N = 3001 d = 96: 2007 -> 20.1 us.  Error against 64
 // bits at the first: 5.9e-7 -> 4.0e-7.  Of the 50 us, MFMAs are 20, K and V
-// reads from LDS about 8, writing and merging the split records about 15.
+// reads from LDS about 8, and the merge launch 4.9.
 #pragma once
 
 #include <math.h>

@@ -341,10 +341,9 @@ DecodePlan make_plan(int B, int Hq, int Hkv, int d, int max_len, bool aligned, b
         splits = std::min<long>(requested, max_len);
         splits = std::min<long>(splits, std::max(max_splits, 1));
         chunk = static_cast<int>((max_len + splits - 1) / splits);
-        // Tuned kernels get chunks of whole workgroup tiles: matrix-core tiles
-        // must start at multiples of 4 tokens (aligned scale quads), and in a
-        // paged cache no wave tile may straddle a page.  So fewer splits than
-        // requested may run.
+        // Tuned kernels get chunks of whole workgroup tiles, so that only a
+        // sequence's last tile is partial and, in a paged cache, no wave tile
+        // straddles a page.  So fewer splits than requested may run.
         if (p.fast && splits > 1) chunk = static_cast<int>(round_up(static_cast<size_t>(chunk), gran));
     } else {
         if (static_cast<long>(max_len) * (2 * d + 8) < kMinSplitUnitBytes)
@@ -605,8 +604,8 @@ bool decode_mfma_layout(const kvq_decode_params* p) {
 
 // The plan of a decode problem.  room: the size of a scratch array that cannot
 // grow (kvq_decode_launch_noalloc).  Padded tiles can need records where the
-// kernels that fill their tiles run without any (a ragged B700 Hq128/Hkv32 d48
-// step: 18 MB against none); a step too large for the array with them takes
+// kernels that fill their tiles run without any (a ragged B700 Hq128/Hkv8 d48
+// step: 19 MB against none); a step too large for the array with them takes
 // the unpadded plan.
 DecodePlan decode_plan(const kvq_decode_params* p, size_t room = SIZE_MAX) {
     auto plan = [&](bool quads, bool padding) {

@@ -16,9 +16,9 @@
 //   into the A operand (lane l: token l%16, dims 16*(l/16) + [0,16) of each
 //   64-dim block); no dequantisation instruction touches K.  q is held as three
 //   balanced int8 limbs of a 22-bit fixed-point value per head (q*2^E rounded
-//   once, |error| <= 2^-23 * max|q|), one MFMA column block per limb; the int32
+//   once, |error| <= 2^-22 * max|q|), one MFMA column block per limb; the int32
 //   products are exact, and dot = ((C0*2^16 + C1*2^8) + C2) * 2^-E.  PAD: four
-//   limbs, 30 bits, which hold every fp32 q to 2^-31 * max|q| (q_limbs).
+//   limbs, 30 bits, which hold q to 2^-30 * max|q| (q_limbs).
 //   MFMA rows n = 0..15 all carry head n % G (duplicates are free).
 // * softmax: the running max m of s = (dot * k_scale) * softmax_scale * log2 e
 //   gives p = exp2(s - m) and the denominator; the PV weights are

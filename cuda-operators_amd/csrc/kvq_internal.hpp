@@ -175,7 +175,7 @@ struct PrefillArgs {
     unsigned max_groups;  // grid cap per plane (0: the default); beyond it workgroups stride
 };
 // vec_ok: 16-byte aligned inputs and 8-byte aligned caches (tuned kernel for
-// d in {32, 64, 128, 256}).
+// rows of whole 16-byte pieces up to 256 elements).
 hipError_t launch_prefill(const PrefillArgs& a, int d, bool bf16, bool vec_ok, hipStream_t stream);
 hipError_t launch_fill_zero(void* p, size_t bytes, hipStream_t stream);
 

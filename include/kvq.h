@@ -36,8 +36,11 @@
 extern "C" {
 #endif
 
-/* Largest head_dim any entry point accepts (32 and multiples of 16 from 48 to
- * 256 run the tuned kernels; any other value up to this bound runs a generic kernel). */
+/* Largest head_dim any entry point but dense attention accepts (there: 1024).
+ * Decode runs tuned kernels at 32 and multiples of 16 from 48 to 256, the
+ * prefill quantiser at multiples of 4 (fp32) or 8 (bf16) up to 256,
+ * kvq_quantize_rows_launch at 32, 64, 128 and 256, dense attention up to 256;
+ * any other value up to the bound runs a generic kernel. */
 #define KVQ_MAX_HEAD_DIM 4096
 
 /* Longest sequence any decode entry point attends to, in tokens: seq_len of
@@ -140,9 +143,12 @@ hipError_t kvq_decode_launch(const kvq_decode_params* p, void* workspace, size_t
  * KVQ_NOALLOC_SCRATCH_BYTES device array that each GPU holds until the process
  * ends (its counters are zero-filled by a kernel on the first call on each
  * device and left at zero by every completed launch).  Same plan, kernels and
- * result bits as kvq_decode_launch.  hipErrorInvalidValue for the arguments
- * kvq_decode_launch rejects and when kvq_decode_workspace_size(p) exceeds
- * KVQ_NOALLOC_SCRATCH_BYTES.  All calls on one GPU share the array: calls that
+ * result bits as kvq_decode_launch while kvq_decode_workspace_size(p) is at most
+ * KVQ_NOALLOC_SCRATCH_BYTES.  Beyond that the call is planned again without
+ * padded tiles (which can need records where other kernels need none: other
+ * kernels and summation order, the same results to rounding);
+ * hipErrorInvalidValue when that plan does not fit either, and for the
+ * arguments kvq_decode_launch rejects.  All calls on one GPU share the array: calls that
  * overlap in time on one GPU (different streams, or host threads) race. */
 hipError_t kvq_decode_launch_noalloc(const kvq_decode_params* p, hipStream_t stream);
 

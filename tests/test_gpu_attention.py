@@ -4,10 +4,10 @@ attention/softmax_new.cu (kvq_ref_attention_f32, pinned in test_oracle.py).
 
 Tolerance: |gpu - oracle| <= 1e-4 + 1e-3 * |oracle| per element (fp32 with a
 different summation order and exp2 of log2-scaled scores).  Cases: the
-matrix-core head dims (32, 64, 128, 256) with query counts around the
-128-query block and key counts around the 64-key tile (32 at d = 256), split and unsplit plans,
-explicit split requests, untuned head dims and misaligned pointers (generic
-kernel), peaked and flat softmax, workspace reuse across calls, a side
+head dims 32, 64, 128 and 256 with query counts around the 64-query block and
+key counts around the 32-key tile, split and unsplit plans, explicit split
+requests, other head dims (the generic kernel above 256) and misaligned pointers
+(generic kernel), peaked and flat softmax, workspace reuse across calls, a side
 stream, and at full prefill size a float64 check of sampled rows."""
 import math
 
@@ -166,9 +166,8 @@ def test_attention_direct_peaked_and_splits(o, d, M, N, splits):
 @pytest.mark.parametrize("M,N", [(1, 1), (1, 4099), (7, 64), (128, 65), (129, 300), (200, 1000), (256, 4096),
                                  (1000, 127), (513, 2048), (63, 1024), (65, 700), (191, 256)])
 def test_attention_online_tuned(o, d, M, N):
-    """Query blocks of 128 (8 waves) where they fill the GPU -- (256, 4096)
-    -- and of 64 (4 waves, d <= 128) where they do not: the other shapes,
-    with rows past M in the last block."""
+    """Few queries, and query blocks of 64 with rows past M in the last one
+    (wider blocks: test_gpu_attention_limbs.py)."""
     rng = np.random.default_rng(M * 7919 + N * 31 + d)
     q, k, v = _problem(rng, M, N, d)
     out = _gpu.poisoned((M, d))

@@ -91,7 +91,7 @@ def paged_decode(q, kp, vp, ksp, vsp, table, lengths, splits=0, k_new=None, v_ne
     return down(out), down(g[1]), down(g[2]), down(g[3]), down(g[4]), dec
 
 
-CASES = [  # (G, d, page): MFMA needs d = 128, G % 4 == 0 and a power-of-two page >= 32;
+CASES = [  # (G, d, page): MFMA takes G >= 2, d a multiple of 16 from 48 to 128 and a power-of-two page >= 16;
     (1, 128, 16), (1, 128, 32), (1, 128, 256),  # the VALU kernel a power-of-two page that is a
     (2, 64, 32), (1, 256, 16), (1, 32, 64),     # multiple of its wave tile; anything else runs
     (4, 128, 32), (8, 128, 128), (4, 128, 64),  # the generic kernel.
