@@ -194,6 +194,65 @@ hipError_t finish_call(hipError_t err, hipStream_t stream) {
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// Steps too small for padded tiles, which cost a fixed time per workgroup
+// (launch, plan, one tile whatever its fill) and pay by reading the cache once;
+// they keep the kernel that fills its tiles or has none.  Times: that kernel /
+// the padded one.
+enum class SmallStep { No, General, Fma, FullTiles };
+SmallStep small_step(int B, int Hkv, int G, int d, int max_len, bool ragged, int sg_m, int sg_v) {
+    const long kv = static_cast<long>(B) * Hkv;
+    const long len = std::max(max_len, 1);
+    if (d == 64 || d == 128) {
+        // Twelve heads (and 20, 28, ..) in full groups of four read the cache
+        // once more than in groups of six: d = 128 Hkv8 B4 L2048 (17 MB) ragged
+        // 17.7 / 20.4 us, B8 L1300 (22 MB) 19.9 / 19.8; uniform B8 L640 (11 MB)
+        // 10.0 / 10.6, B4 L1300 13.1 / 11.8, d = 64 B8 L1300 11.4 / 12.0.
+        if (sg_m > 0 && G > 8 && G % 8 == 4)
+            return kv * len * (2 * d + 8) < (ragged ? 20L << 20 : 10L << 20) ? SmallStep::FullTiles : SmallStep::No;
+        // Odd groups: one head per FMA workgroup of eight waves, where the
+        // matrix-core plan has one workgroup of four (G = 7 d = 128 L384 7.2 /
+        // 8.5 us, d = 64 L900 7.7 / 9.4; L640 7.2 / 7.6, G = 3 7.5 / 6.9; G = 7
+        // d = 64 Hkv8 B4 L900, 224 workgroups, 10.5 / 9.8), or ragged lengths
+        // within one FMA tile, planned in the kernel (G = 7 d = 64 L192 Hkv8 B4 8.3 /
+        // 9.5 us, B8 10.1 / 9.8; d = 128 L64 7.3 / 8.7; L192, two tiles, 13.6 / 11.1).
+        if (sg_m > 0 && sg_v == 1 && G > 1) {
+            const long unit = len * (2 * d + 8);
+            const bool one_tile = len <= kvq::fast_tile_tokens(d, 1) && (d == 128 || len > 128);
+            if (ragged ? one_tile && B <= kvq::kFitMaxSeqs && kv * G <= 256 : unit >= 96 * 1024 && unit < kMinSplitUnitBytes && kv * G <= 64)
+                return SmallStep::Fma;
+        }
+        return SmallStep::No;
+    }
+    if (d == 32 || d == 256) return SmallStep::No;
+    // Other head dims: short sequences in large batches, where the general
+    // kernel's time per token is less than a padded workgroup's fixed time.
+    // Estimates in ns, fitted to the times below (launches cannot follow each
+    // other in less than 7 us): general, a wave per query head, its chain of
+    // tokens or the chip's throughput; padded, by workgroups.
+    const long passes = (d + 63) / 64;
+    const long heads = kv * G;
+    const long chip = len * heads * (60 + 70 * passes) / 1000;
+    const long general = std::max({7000L, 3000 + len * (300 + 170 * passes), passes >= 3 ? chip * 3 / 2 : chip});
+    long padded;
+    if (sg_m > 0) {
+        // Uniform d = 48, 3 heads, Hkv8 B256: L12 12.3 / 15 us, B1000 L12 45 / 52,
+        // L16 55 / 52; d = 112 B256 L12 16 / 21, L16 24 / 21; d = 80, 8 heads, Hkv4
+        // B256 L4 9.6 / 12.8, L8 13.3 / 12.8; ragged d = 112 B256 L4 8.5 / 13.3, L8
+        // 11.6 / 13.5, d = 48 L8 9.8 / 10, L12 12.5 / 10.5, B1000 L4 18 / 25, L8 30 / 26.
+        const long groups = kv * ((G + sg_m - 1) / sg_m);
+        padded = 2000 + groups * (ragged ? (d <= 64 ? 3000 : 4500) : (d <= 64 ? 6300 : 9500)) / 1000;
+    } else {
+        // Uniform d = 48 Hkv8 B256: L24 15.6 / 19.6 us, L32 19.6 / 19.9, B1000 L48 52 /
+        // 66, L64 72 / 67; d = 96 Hkv32 B64 L16 14.5 / 18.4, L24 20 / 18.7, B256 L32
+        // 55 / 63; d = 240 Hkv8 B256 L12 17.2 / 17.7, L16 32 / 17.8; d = 144, 2 heads,
+        // B256 L16 21 / 38, L24 45 / 40; d = 192, 4 heads, Hkv4 B256 L16 31 / 35, L24
+        // 50 / 37; ragged d = 192 B1 L4 6.9 / 13.2, L12 13.1 / 13.3, B64 L12 13.9 / 22.6.
+        padded = 2000 + 8 * heads + (!ragged ? 0 : B > 64 ? 4000 : 100L * B + (sg_v == 4 ? 3000 : 0));
+        if (sg_v == 4) padded = std::max(padded, 9800L);
+    }
+    return general < std::max(padded, 7000L) ? SmallStep::General : SmallStep::No;
+}
+
 // Split count and workspace layout for one decode problem.
 // aligned: q, caches and new rows are 16-byte aligned (vector loads);
 // quads: the matrix-core kernel's layout needs hold (scale arrays 4-byte
@@ -209,11 +268,17 @@ DecodePlan make_plan(int B, int Hq, int Hkv, int d, int max_len, bool aligned, b
                      bool ragged, int requested, int max_splits, bool fused, bool padding = true) {
     DecodePlan p{};
     const int G = Hq / Hkv;
-    const int sg_m = padding                            ? kvq::mfma_heads_per_group(G, d)
-                     : (d != 64 && d != 128) || G % 4 != 0 ? 0
-                     : G % 8 == 0                          ? 8
-                                                           : 4;
+    int sg_m = padding                            ? kvq::mfma_heads_per_group(G, d)
+               : (d != 64 && d != 128) || G % 4 != 0 ? 0
+               : G % 8 == 0                          ? 8
+                                                     : 4;
     const int sg_v = kvq::fast_heads_per_group(G);
+    if (padding && requested == 0) {
+        const SmallStep s = small_step(B, Hkv, G, d, max_len, ragged, sg_m, sg_v);
+        if (s == SmallStep::General) aligned = false;
+        if (s == SmallStep::Fma) sg_m = 0;
+        if (s == SmallStep::FullTiles) sg_m = 4;
+    }
     const bool pow2 = page > 0 && (page & (page - 1)) == 0;
     const int wave_tokens = kvq::fast_wave_tokens(d, sg_v);
     const bool valu_pages = page == 0 || (pow2 && wave_tokens > 0 && page % wave_tokens == 0);

@@ -472,6 +472,37 @@ def test_decode_plan_kernels(L):
     assert plan(1, 4, 4, 128, 8192, splits=8).splits == 8
 
 
+def test_decode_plan_of_small_steps(L):
+    """Steps too small for padded tiles keep the kernel that fills its tiles:
+    short sequences in large batches the general kernel, twelve heads per kv head
+    full groups of four, odd groups over few keys the FMA kernel; the same shapes
+    with more tokens run padded."""
+    A = 1 << 20
+
+    def plan(B, Hq, Hkv, d, n, ragged=False):
+        return kvq.decode_plan(kvq.DecodeParams(B, Hq, Hkv, d, n, n, A if ragged else None, A, A, A, A, A, A, 0.0, 0,
+                                                None, None))
+
+    for B, G, Hkv, d, short, long, padded in ((1000, 4, 2, 192, 2, 130, kvq.KERNEL_DECODE_VALU),
+                                              (256, 1, 32, 96, 8, 64, kvq.KERNEL_DECODE_VALU),
+                                              (1000, 3, 8, 48, 4, 24, kvq.KERNEL_DECODE_MFMA),
+                                              (1000, 16, 2, 80, 2, 24, kvq.KERNEL_DECODE_MFMA)):
+        for ragged in (False, True):
+            assert plan(B, G * Hkv, Hkv, d, short, ragged).kernel == kvq.KERNEL_DECODE_GENERIC
+            assert plan(B, G * Hkv, Hkv, d, long, ragged).kernel == padded
+    for d in (64, 128):
+        for ragged in (False, True):
+            assert plan(4, 96, 8, d, 640, ragged).heads_per_group == 4
+            assert plan(16, 96, 8, d, 8192, ragged).heads_per_group == 6
+    assert plan(4, 96, 8, 96, 640).heads_per_group == 6  # no full tiles at other head dims
+    for d, n, big in ((64, 900, 4096), (128, 384, 4096)):
+        assert plan(1, 7, 1, d, n).kernel == kvq.KERNEL_DECODE_VALU
+        assert plan(1, 7, 1, d, big).kernel == plan(64, 56, 8, d, n).kernel == kvq.KERNEL_DECODE_MFMA
+    for d, n in ((64, 256), (128, 128)):
+        assert plan(4, 56, 8, d, n, True).kernel == kvq.KERNEL_DECODE_VALU
+        assert plan(4, 56, 8, d, n + 1, True).kernel == plan(16, 56, 8, d, n, True).kernel == kvq.KERNEL_DECODE_MFMA
+
+
 def test_attention_plan_routes_misaligned_to_generic(L):
     """Unaligned q/k/v/out at a tuned head dim take attention_generic, unsplit
     (the tuned kernels use 16-byte vector accesses)."""
