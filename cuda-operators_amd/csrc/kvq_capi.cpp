@@ -662,7 +662,7 @@ bool aligned4(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 3u) == 0
 // buffer resource with 32-bit byte offsets (capacity * head_dim < 2^31).  Its
 // loads of 4 consecutive scales need 4-byte alignment only, and the dwords of
 // a quad past the end of the row read 0 one by one, so the capacity may be odd
-// (B4 Hq32/Hkv8 d128 of 130 tokens: 12.0 us in the FMA kernel, 5.6 us).
+// (B4 Hq32/Hkv8 d128 of 130 tokens: 12.2 us in the FMA kernel, 7.6 us).
 bool decode_mfma_layout(const kvq_decode_params* p) {
     return aligned4(p->k_scale) && aligned4(p->v_scale) && p->capacity < (1 << 24);
 }

@@ -1486,6 +1486,10 @@ __global__ __launch_bounds__(kMWaves* kWave) __attribute__((amdgpu_waves_per_eu(
 int mfma_tile_tokens() { return kMBStep; }
 
 // Heads per workgroup: G heads in ceil(G / 8) groups as equal as they come.
+// Two heads already read the cache once in place of once per head (the FMA
+// kernel's two-head workgroups take as long from 16 tokens up, uniform and
+// ragged: Hkv8 d = 128 B1 L512 9.9 / 8.3 us, B8 L4096 21.9 / 16.1, B64 L4096 105 /
+// 83, B256 L512 80 / 51; d = 64 B32 L2048 19.3 / 16.0).
 int mfma_heads_per_group(int G, int d) {
     if (G < 2 || d % 16 != 0 || d < 48 || d > 128) return 0;
     const int groups = (G + 7) / 8;
