@@ -273,12 +273,6 @@ DecodePlan make_plan(int B, int Hq, int Hkv, int d, int max_len, bool aligned, b
                : G % 8 == 0                          ? 8
                                                      : 4;
     const int sg_v = kvq::fast_heads_per_group(G);
-    if (padding && requested == 0) {
-        const SmallStep s = small_step(B, Hkv, G, d, max_len, ragged, sg_m, sg_v);
-        if (s == SmallStep::General) aligned = false;
-        if (s == SmallStep::Fma) sg_m = 0;
-        if (s == SmallStep::FullTiles) sg_m = 4;
-    }
     const bool pow2 = page > 0 && (page & (page - 1)) == 0;
     const int wave_tokens = kvq::fast_wave_tokens(d, sg_v);
     const bool valu_pages = page == 0 || (pow2 && wave_tokens > 0 && page % wave_tokens == 0);
@@ -287,7 +281,14 @@ DecodePlan make_plan(int B, int Hq, int Hkv, int d, int max_len, bool aligned, b
     const int force = forced_kernel();
     if (force == kForceGeneric) aligned = false;
     if (force == kForceValu) quads = false;
-    if (aligned && quads && mfma_pages && sg_m > 0) {
+    if (!quads || !mfma_pages) sg_m = 0;
+    if (padding && requested == 0) {
+        const SmallStep s = small_step(B, Hkv, G, d, max_len, ragged, sg_m, sg_v);
+        if (s == SmallStep::General) aligned = false;
+        if (s == SmallStep::Fma && valu_pages) sg_m = 0;
+        if (s == SmallStep::FullTiles) sg_m = 4;
+    }
+    if (aligned && sg_m > 0) {
         p.kernel = kvq::Kernel::Mfma;
         p.sg = sg_m;
         tile = kvq::mfma_tile_tokens();

@@ -503,6 +503,18 @@ def test_decode_plan_of_small_steps(L):
         assert plan(4, 56, 8, d, n + 1, True).kernel == plan(16, 56, 8, d, n, True).kernel == kvq.KERNEL_DECODE_MFMA
 
 
+def test_paged_plan_of_small_steps(L):
+    """The FMA kernel takes a small ragged step of an odd group only from pages
+    its wave tiles fit in (32 tokens at d = 64, 16 at d = 128)."""
+    A = 1 << 20
+    for d, page, n, kernel in ((64, 16, 192, kvq.KERNEL_DECODE_MFMA), (64, 32, 192, kvq.KERNEL_DECODE_VALU),
+                               (128, 16, 112, kvq.KERNEL_DECODE_VALU), (64, 48, 192, kvq.KERNEL_DECODE_GENERIC)):
+        p = kvq.PagedDecodeParams(batch=4, num_q_heads=14, num_kv_heads=2, head_dim=d, page_size=page, num_pages=64,
+                                  max_pages_per_seq=n // page, max_seq_len=0, block_table=A, lengths=A, q=A, k_pages=A,
+                                  v_pages=A, k_scale_pages=A, v_scale_pages=A, out=A)
+        assert kvq.paged_decode_plan(p).kernel == kernel, (d, page)
+
+
 def test_attention_plan_routes_misaligned_to_generic(L):
     """Unaligned q/k/v/out at a tuned head dim take attention_generic, unsplit
     (the tuned kernels use 16-byte vector accesses)."""
